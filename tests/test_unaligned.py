@@ -1,0 +1,100 @@
+"""Tensors without the 16-byte vector layout: head dims that are no multiple of 8, V^T rows of an
+odd key count, bases at any element. The kernels read such rows 16 bytes at a time, the pieces at a
+row's end as its last eight elements; each case here ends rows, tiles or tensors inside a piece.
+Inputs lie between NaN guards (a value taken from outside a tensor makes the output NaN) and O
+between guards that must survive."""
+import numpy as np
+import pytest
+
+import transfer_station_amd as ts
+
+pytestmark = pytest.mark.gpu
+
+PAD = 32  # guard elements on each side
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu_present():
+    assert ts.device_count() >= 1, "no HIP device visible: GPU tests must run on the MI355X box"
+
+
+def guarded(arr, off):
+    """(buffer, address of arr's copy in it), off elements past a 16-byte boundary."""
+    full = np.full(arr.size + 2 * PAD + off, 0xFFFF, np.uint16)
+    full[PAD + off:PAD + off + arr.size] = arr
+    buf = ts.DeviceBuffer.from_array(full)
+    return buf, buf.ptr + 2 * (PAD + off)
+
+
+def attend(Q, K, V, Hq, Hkv, Sq, Sk, D, causal, vt, off):
+    n = Hq * Sq * D
+    bufs = [guarded(a, off) for a in (Q, K, V)]
+    with ts.DeviceBuffer(4 * (n + 2 * PAD)) as do, \
+            ts.DeviceBuffer(ts.attn_flash_scratch_bytes(D, 128)) as ds:
+        do.fill_bytes(0xFF)
+        ds.fill_bytes(0xFF)
+        ts.attn_flash(bufs[0][1], bufs[1][1], bufs[2][1], do.ptr + 4 * PAD, Hq, Hkv, Sq, Sk, D,
+                      causal, 128, ds, vt)
+        ts.synchronize()
+        raw = do.download(np.uint32)
+    for b, _ in bufs:
+        b.free()
+    assert np.all(raw[:PAD] == 0xFFFFFFFF) and np.all(raw[PAD + n:] == 0xFFFFFFFF)
+    return raw[PAD:PAD + n].view(np.float32)
+
+
+CASES = [
+    # Hq, Hkv, Sq, Sk, D, causal, base offset in elements
+    (4, 2, 70, 65, 7, 1, 0),          # rows shorter than a piece
+    (4, 2, 70, 129, 9, 0, 0),         # one whole piece and one element
+    (6, 3, 130, 257, 65, 1, 0),       # 96-wide tiles, key halves, a one-key last tile
+    (8, 2, 200, 1023, 100, 0, 0),     # key split: partials of a head dim that is no multiple of 8
+    (8, 2, 500, 501, 127, 1, 0),      # causal key split at DP = 128
+    (160, 40, 300, 255, 100, 0, 0),   # 8 waves, ragged query and key tails
+    (136, 34, 520, 521, 81, 1, 0),    # 8 waves, causal, DP = 96
+    (40, 40, 1000, 70, 63, 1, 0),     # Sq > Sk: rows that attend nothing
+    (32, 8, 20, 333, 44, 1, 0),       # packed short query blocks
+    (4, 2, 140, 100, 129, 1, 0),      # 256-wide tiles
+    (2, 1, 33, 63, 255, 0, 0),
+    (8, 2, 150, 260, 128, 1, 1),      # the vector layout but for the bases: 2-byte aligned
+    (64, 16, 300, 200, 64, 0, 3),
+    (8, 2, 140, 7, 128, 0, 0),        # V^T rows shorter than a piece
+    (4, 2, 140, 9, 40, 1, 0),
+    (32, 8, 1, 1001, 100, 0, 0),      # decode, split
+    (8, 2, 5, 517, 33, 1, 1),         # decode, three row blocks
+    (64, 64, 1, 2309, 128, 0, 5),     # decode, V^T groups of four steps and a one-key tail
+    (4, 2, 3, 5, 128, 1, 0),          # decode, V^T rows shorter than a piece
+    (4, 2, 2, 40, 5, 0, 0),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=["-".join(map(str, c)) for c in CASES])
+def test_unaligned(oracle, case):
+    Hq, Hkv, Sq, Sk, D, causal, off = case
+    print("case", case, flush=True)
+    Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, 991 + D)
+    Vt = np.ascontiguousarray(V.reshape(Hkv, Sk, D).transpose(0, 2, 1)).ravel()
+    rows = oracle.ref_rowset(Sq, 16)
+    R = oracle.attn_ref(Q, K, V, Hq, Hkv, Sq, Sk, D, causal, rows, nthreads=8)
+    for vt in (0, 1):
+        O = attend(Q, K, Vt if vt else V, Hq, Hkv, Sq, Sk, D, causal, vt, off)
+        # the reference's pass rule; P rounded to bf16 (2^-9 of a weight) stays well below it
+        ok, mad, maxref, nbad = oracle.cmp_rows(R, O, Hq, Sq, D, rows)
+        print("   vt=%d err/scale=%.2e nbad=%d" % (vt, mad / maxref, nbad), flush=True)
+        assert ok and nbad == 0, (case, vt, mad, maxref)
+
+
+@pytest.mark.parametrize("Hkv,Sk,D", [(3, 129, 65), (2, 1, 300), (1, 260, 7), (2, 135, 64),
+                                      (1, 7, 128), (5, 128, 70)])
+def test_unaligned_pack(Hkv, Sk, D):
+    V = np.arange(Hkv * Sk * D, dtype=np.uint32).astype(np.uint16)
+    src, addr = guarded(V, 1)
+    dst, out = guarded(np.zeros(V.size, np.uint16), 3)
+    ts.pack_v_full(addr, out, Hkv, Sk, D)
+    ts.synchronize()
+    raw = dst.download(np.uint16)
+    got = raw[PAD + 3:PAD + 3 + V.size].reshape(Hkv, D, Sk)
+    assert np.array_equal(got, V.reshape(Hkv, Sk, D).transpose(0, 2, 1))
+    assert np.all(raw[:PAD + 3] == 0xFFFF) and np.all(raw[PAD + 3 + V.size:] == 0xFFFF)
+    src.free()
+    dst.free()

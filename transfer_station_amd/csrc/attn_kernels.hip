@@ -12,21 +12,20 @@
 // products s, p = 2^(s*c - m*c) equals e^(scale*s - scale*m).
 //
 // Kernels:
-//   attn_prefill_fast_kernel<DP,KT,NW,CAUSAL,VT,KH>  MFMA prefill for D % 8 == 0, D <= DP in
-//                                          {64, 96, 128, 256}; one workgroup = NW waves x 32 rows,
-//                                          or (KH) 8 waves over 128 rows on key-tile halves
+//   attn_prefill_fast_kernel<DP,KT,NW,CAUSAL,VT,KH,UA>  MFMA prefill, D <= DP in {64, 96, 128,
+//                                          256}; one workgroup = NW waves x 32 rows, or (KH) 8
+//                                          waves over 128 rows on key-tile halves; UA: tensors
+//                                          without the 16-byte vector layout
 //   attn_prefill_persist_kernel<DP,CAUSAL,KH> the same tile code at D <= 128, one 8-wave
 //                                          workgroup per CU running its 256-row items back to
 //                                          back (causal: pairs of a heavy and a light query
 //                                          tile), or (KH) one causal pair of 128-row items on
 //                                          key-tile halves
-//   attn_prefill_kernel<DP,KT,CAUSAL,VEC,VT> the same tiling for any D <= 256 and alignment
 //   attn_decode_kernel<DP,CAUSAL,VEC,VT>   split-K decode for g*Sq <= 64 rows per kv head
-//   attn_decode_vt_kernel<DP,CAUSAL>       the same from V^T, staged in LDS 512 keys at a time
+//   attn_decode_vt_kernel<DP,CAUSAL,NTL,UA> the same from V^T, staged in LDS 512 keys at a time
 //   attn_merge{2,w,}_kernel                log-sum-exp merge of split partials (2 splits / up to
 //                                          64, one wave per row / any, one workgroup per row)
-//   attn_pack_v16_kernel / attn_pack_v_kernel  V [Hkv][Sk][D] -> V^T [Hkv][D][Sk] (16-byte
-//                                          vector path / any shape)
+//   attn_pack_v16_kernel<TK,VEC>           V [Hkv][Sk][D] -> V^T [Hkv][D][Sk]
 // VT selects a pre-transposed V ([Hkv][D][Sk], pack_v_full's layout).
 #include <hip/hip_runtime.h>
 #include <stdarg.h>
@@ -69,7 +68,6 @@ __device__ __forceinline__ int wg_id_x() { return (int)__builtin_amdgcn_workgrou
 __device__ __forceinline__ int wg_id_y() { return (int)__builtin_amdgcn_workgroup_id_y(); }
 __device__ __forceinline__ int wg_id_z() { return (int)__builtin_amdgcn_workgroup_id_z(); }
 __device__ __forceinline__ int wi_id_x() { return (int)__builtin_amdgcn_workitem_id_x(); }
-__device__ __forceinline__ int wi_id_y() { return (int)__builtin_amdgcn_workitem_id_y(); }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (each with its own L2). Remap the
 // hardware block id so that consecutive logical ids land on the same XCD: logical ids that
@@ -109,44 +107,84 @@ __device__ __forceinline__ u32x4 zero4() {
     return z;
 }
 
+// Unaligned vectors: gfx950 serves 16-byte global accesses at any element alignment, so tensors
+// whose rows are not 16-byte aligned are read 16 bytes at a time too (element-wise loads, eight
+// 2-byte loads and their packing per chunk, made such calls 6-15x slower). O is fp32: 4-aligned.
+typedef u32x4 __attribute__((aligned(2))) u32x4_a2;
+typedef f32x4 __attribute__((aligned(4))) f32x4_a4;
+
+template <bool NT> __device__ __forceinline__ u32x4 load16_any(const uint16_t *p) {
+    return NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2 *>(p))
+              : *reinterpret_cast<const u32x4_a2 *>(p);
+}
+
+// v without its first n (0..8) of eight 16-bit elements, zeros behind.
+__device__ __forceinline__ u32x4 drop_elems(u32x4 v, int n) {
+    const int h = (n & 1) * 16;
+    const bool n2 = n & 2, n4 = n & 4, n8 = n & 8;
+    const uint32_t a0 = __builtin_amdgcn_alignbit(v[1], v[0], h);
+    const uint32_t a1 = __builtin_amdgcn_alignbit(v[2], v[1], h);
+    const uint32_t a2 = __builtin_amdgcn_alignbit(v[3], v[2], h), a3 = v[3] >> h;
+    const uint32_t b0 = n2 ? a1 : a0, b1 = n2 ? a2 : a1, b2 = n2 ? a3 : a2, b3 = n2 ? 0u : a3;
+    return u32x4{n8 ? 0u : n4 ? b2 : b0, n8 ? 0u : n4 ? b3 : b1, n4 || n8 ? 0u : b2,
+                 n4 || n8 ? 0u : b3};
+}
+
+// Elements [i, i+8) of the n-element row at p, zero-filled past n, at any alignment and without a
+// read outside the row: a chunk that reaches past the row's end is read as its last eight
+// elements and shifted. may (wave-uniform) false: the caller knows that no chunk does. SHORT: the
+// row may have fewer than eight elements.
+template <bool NT = false, bool SHORT = true>
+__device__ __forceinline__ u32x4 load_run8(const uint16_t *p, int i, int n, bool may) {
+    if (!may)
+        return load16_any<NT>(p + i);
+    if (SHORT && n < 8) { // a row shorter than a chunk: element by element, rolled (rare)
+        u32x4 v = zero4();
+#pragma unroll 1
+        for (int j = min(n, i + 8) - 1; j >= i; --j)
+            v = u32x4{(v[0] << 16) | p[j], __builtin_amdgcn_alignbit(v[1], v[0], 16),
+                      __builtin_amdgcn_alignbit(v[2], v[1], 16),
+                      __builtin_amdgcn_alignbit(v[3], v[2], 16)};
+        return v;
+    }
+    const int back = min(max(i + 8 - n, 0), 8);
+    return drop_elems(load16_any<NT>(p + min(i, n - 8)), back);
+}
+
 // Eight consecutive bf16 of one row, columns [col, col+8), zero-filled past D or when !ok.
-// VEC requires D % 8 == 0 and a 16-byte aligned base, so one 16-byte load covers them.
+// VEC requires D % 8 == 0 and a 16-byte aligned base, so one 16-byte load covers them; otherwise
+// ce (wave-uniform) bounds the columns of the wave's lanes, so that only a chunk column that
+// reaches past D pays for the shift.
 // NT marks the load non-temporal (data read once: HBM streams such loads ≈ 15% faster).
-template <bool VEC, bool NT = false>
+template <bool VEC, bool NT = false, bool SHORT = true>
 __device__ __forceinline__ u32x4 load_row8(const uint16_t *base, size_t row, int col, int D,
-                                           bool ok) {
+                                           bool ok, int ce = 0x7fffffff) {
     if (!ok || col >= D)
         return zero4();
-    const uint16_t *p = base + row * (size_t)D + col;
-    if (VEC)
-        return NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p))
-                  : *reinterpret_cast<const u32x4 *>(p);
-    uint32_t e[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-        e[j] = (col + j < D) ? (uint32_t)p[j] : 0u;
-    u32x4 r = {e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-    return r;
+    const uint16_t *p = base + row * (size_t)D;
+    if (!VEC)
+        return load_run8<NT, SHORT>(p, col, D, (D & 7) != 0 && ce > D);
+    p += col;
+    return NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p))
+              : *reinterpret_cast<const u32x4 *>(p);
 }
 
 // Eight consecutive keys [key, key+8) of row d of a V^T head ([D][Sk], row stride Sk), zero-filled
 // at d >= D or key >= klim. VEC requires Sk % 8 == 0 (with key % 8 == 0 and klim % 8 == 0 a chunk
-// is then wholly inside or wholly outside) and a 16-byte aligned base.
+// is then wholly inside or wholly outside) and a 16-byte aligned base; otherwise ke
+// (wave-uniform) bounds the keys of the wave's lanes, and klim is a multiple of 8 above key or Sk
+// (the row's end), as for the keys of a tile.
 template <bool VEC, bool NT = false>
 __device__ __forceinline__ u32x4 load_vt8(const uint16_t *base, int d, int key, int Sk, int D,
-                                          int klim) {
+                                          int klim, int ke = 0x7fffffff) {
     if (d >= D || key >= klim)
         return zero4();
-    const uint16_t *p = base + (size_t)d * Sk + key;
-    if (VEC)
-        return NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p))
-                  : *reinterpret_cast<const u32x4 *>(p);
-    uint32_t e[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-        e[j] = (key + j < klim) ? (uint32_t)p[j] : 0u;
-    u32x4 r = {e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-    return r;
+    const uint16_t *p = base + (size_t)d * Sk;
+    if (!VEC)
+        return load_run8<NT>(p, key, klim, ke > klim);
+    p += key;
+    return NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p))
+              : *reinterpret_cast<const u32x4 *>(p);
 }
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
@@ -207,8 +245,10 @@ __device__ __forceinline__ void lds_wave_fence() {
 }
 
 // ------------------------------------------------------------------------------------------
-// Prefill. Workgroup = 4 waves; wave w owns query rows q0 = qt*128 + 32w .. +31 of query head h.
-// Per key tile of KT keys (one online-softmax update per tile):
+// Prefill, D <= DP (64, 96, 128 or 256); the head-dim columns D .. DP-1 are zero in the tiles and
+// in Q, and are never stored. NW waves per workgroup (8: 256 query rows, two waves per SIMD; 4 on
+// grids too small to fill the GPU, and always at DP = 256, where one wave per SIMD holds O and Q);
+// wave w owns 32 query rows. Per key tile of KT keys (one online-softmax update per tile):
 //   S^T[key][q] = K_tile . Q^T     (v_mfma_f32_32x32x16_bf16, A = K rows from LDS, B = Q regs)
 //   each lane holds one query (q = lane%32) and 16 keys per 32-key sub-tile, so the row max is
 //   an in-lane reduction plus one exchange with lane^32;
@@ -219,222 +259,7 @@ __device__ __forceinline__ void lds_wave_fence() {
 // VT: V arrives pre-transposed ([Hkv][D][Sk], pack_v_full's output). The tile is then staged
 // d-major (DP rows of KT keys), and the V^T operand of the P.V MFMA is a plain 16-byte LDS read
 // of 8 consecutive keys of one d row; the operand values, and so the result, are the same.
-// ------------------------------------------------------------------------------------------
-template <int DP, int KT, bool CAUSAL, bool VEC, bool VT>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(
-    const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
-    const uint16_t *__restrict__ V, float *__restrict__ O, int Hq, int Hkv, int Sq, int Sk, int D,
-    float c, int nqt) {
-    static_assert(DP % 32 == 0 && KT % 32 == 0, "tile shape");
-    constexpr int KSTR = DP + 8;  // LDS row stride (elements) of K: 16-byte pad
-    constexpr int VSTR = DP + 16; // LDS row stride of V: 32-byte pad
-    constexpr int VTSTR = KT + 8; // LDS row stride of a V^T tile (VT): 16-byte pad
-    constexpr int NCH = KT * DP / 8 / 256; // 16-byte chunks per thread per tile, per tensor
-    static_assert(NCH >= 1 && (KT * DP / 8) % 256 == 0, "chunking");
-    __shared__ __attribute__((aligned(16))) uint16_t Ks[2][KT * KSTR];
-    __shared__ __attribute__((aligned(16))) uint16_t Vs[2][VT ? DP * VTSTR : KT * VSTR];
-
-    const int g = Hq / Hkv;
-    const int L = xcd_remap(wg_id_x(), Hq * nqt); // the grid is Hq * nqt workgroups
-    const int u = L / (g * nqt);
-    const int rr = L - u * (g * nqt);
-    const int qt = rr / g;
-    const int h = u * g + (rr - qt * g);
-
-    const int tid = wi_id_x(), w = tid >> 6, lane = tid & 63;
-    const int l32 = lane & 31, hi = lane >> 5;
-    const int q0 = qt * 128 + w * 32;
-    const int myq = q0 + l32;
-
-    const uint16_t *Qh = Q + (size_t)h * Sq * D;
-    const uint16_t *Kh = K + (size_t)u * Sk * D;
-    const uint16_t *Vh = V + (size_t)u * Sk * D;
-
-    // Q as the B operand: lane holds Q[myq][16kk + 8hi .. +7].
-    bf16x8 qb[DP / 16];
-#pragma unroll
-    for (int kk = 0; kk < DP / 16; ++kk)
-        qb[kk] = as_bf16x8(load_row8<VEC>(Qh, (size_t)myq, kk * 16 + hi * 8, D, myq < Sq));
-
-    // Key tiles this workgroup needs, and the last key any row of this wave may attend.
-    int nkt = (Sk + KT - 1) / KT;
-    int wave_maxkey = (q0 < Sq) ? Sk - 1 : -1;
-    if (CAUSAL) {
-        const int last_row = min(qt * 128 + 127, Sq - 1);
-        const int maxkey = Sk - Sq + last_row;
-        nkt = (maxkey < 0) ? 0 : min(nkt, maxkey / KT + 1);
-        if (q0 < Sq)
-            wave_maxkey = min(Sk - 1, Sk - Sq + min(q0 + 31, Sq - 1));
-    }
-    const int lim = CAUSAL ? min(Sk - 1, Sk - Sq + myq) : Sk - 1;
-
-    float m_run = kNegInf, l_run = 0.f;
-    f32x16 o[DP / 32];
-#pragma unroll
-    for (int db = 0; db < DP / 32; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            o[db][i] = 0.f;
-
-    u32x4 kr[NCH], vr[NCH];
-    auto gload = [&](int kt) {
-#pragma unroll
-        for (int r = 0; r < NCH; ++r) {
-            const int cidx = tid + 256 * r;
-            const int row = cidx / (DP / 8), col = (cidx % (DP / 8)) * 8;
-            const int key = kt * KT + row;
-            kr[r] = load_row8<VEC>(Kh, (size_t)key, col, D, key < Sk);
-            if (VT) {
-                const int d = cidx / (KT / 8), kc = (cidx % (KT / 8)) * 8;
-                vr[r] = load_vt8<VEC>(Vh, d, kt * KT + kc, Sk, D, Sk);
-            } else {
-                vr[r] = load_row8<VEC>(Vh, (size_t)key, col, D, key < Sk);
-            }
-        }
-    };
-    auto swrite = [&](int buf) {
-#pragma unroll
-        for (int r = 0; r < NCH; ++r) {
-            const int cidx = tid + 256 * r;
-            const int row = cidx / (DP / 8), col = (cidx % (DP / 8)) * 8;
-            *reinterpret_cast<u32x4 *>(&Ks[buf][row * KSTR + col]) = kr[r];
-            if (VT) {
-                const int d = cidx / (KT / 8), kc = (cidx % (KT / 8)) * 8;
-                *reinterpret_cast<u32x4 *>(&Vs[buf][d * VTSTR + kc]) = vr[r];
-            } else {
-                *reinterpret_cast<u32x4 *>(&Vs[buf][row * VSTR + col]) = vr[r];
-            }
-        }
-    };
-
-    // Row of the K tile this lane feeds to the S^T MFMA (bits 2,3 of l32 swapped).
-    const int kperm = (l32 & ~12) | ((l32 & 4) << 1) | ((l32 & 8) >> 1);
-    const int g16 = lane >> 4, i16 = lane & 15;
-
-    if (nkt > 0) {
-        gload(0);
-        swrite(0);
-    }
-    __syncthreads();
-    for (int kt = 0; kt < nkt; ++kt) {
-        const int buf = kt & 1;
-        if (kt + 1 < nkt)
-            gload(kt + 1);
-        const int kbase = kt * KT;
-        if (kbase <= wave_maxkey) {
-            f32x16 s[KT / 32];
-#pragma unroll
-            for (int t = 0; t < KT / 32; ++t) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    s[t][i] = 0.f;
-                const uint16_t *kb = &Ks[buf][(t * 32 + kperm) * KSTR + hi * 8];
-#pragma unroll
-                for (int kk = 0; kk < DP / 16; ++kk) {
-                    const bf16x8 a = as_bf16x8(*reinterpret_cast<const u32x4 *>(kb + kk * 16));
-                    s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qb[kk], s[t], 0, 0, 0);
-                }
-            }
-            // Register (t, i) of this lane holds key kbase + 32t + 16(i/8) + 8hi + i%8.
-            const bool need_mask =
-                (kbase + KT > Sk) || (CAUSAL && kbase + KT - 1 > Sk - Sq + q0);
-            if (need_mask) {
-#pragma unroll
-                for (int t = 0; t < KT / 32; ++t)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const int key = kbase + t * 32 + 16 * (i >> 3) + 8 * hi + (i & 7);
-                        if (key > lim)
-                            s[t][i] = kNegInf;
-                    }
-            }
-            float mx = kNegInf;
-#pragma unroll
-            for (int t = 0; t < KT / 32; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    mx = fmaxf(mx, s[t][i]);
-            mx = max_xor32(mx);
-            const float mnew = fmaxf(m_run, mx);
-            const float muse = (mnew == kNegInf) ? 0.f : mnew;
-            const float alpha = fast_exp2((m_run - muse) * c);
-            const float mc = muse * c;
-            float psum = 0.f;
-            bf16x8 pk[KT / 16];
-#pragma unroll
-            for (int t = 0; t < KT / 32; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const float p = fast_exp2(fmaf(s[t][i], c, -mc));
-                    psum += p;
-                    pk[2 * t + (i >> 3)][i & 7] = (__bf16)p;
-                }
-            l_run = alpha * l_run + psum;
-            m_run = mnew;
-#pragma unroll
-            for (int db = 0; db < DP / 32; ++db)
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    o[db][i] *= alpha;
-#pragma unroll
-            for (int cc = 0; cc < KT / 16; ++cc) {
-                if (VT) {
-                    // lane: d row 32db + l32, keys 16cc + 8hi .. +7 (the k index of pk[cc]).
-                    const uint16_t *vb = &Vs[buf][l32 * VTSTR + cc * 16 + 8 * hi];
-#pragma unroll
-                    for (int db = 0; db < DP / 32; ++db) {
-                        const bf16x8 a =
-                            as_bf16x8(*reinterpret_cast<const u32x4 *>(vb + db * 32 * VTSTR));
-                        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pk[cc], o[db], 0, 0, 0);
-                    }
-                } else {
-                    const uint16_t *vb = &Vs[buf][(cc * 16 + 8 * hi + (i16 >> 2)) * VSTR +
-                                                  (g16 & 1) * 16 + 4 * (i16 & 3)];
-#pragma unroll
-                    for (int db = 0; db < DP / 32; ++db) {
-                        const bf16x8 a = join_tr(lds_read_tr(vb + db * 32),
-                                                 lds_read_tr(vb + db * 32 + 4 * VSTR));
-                        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pk[cc], o[db], 0, 0, 0);
-                    }
-                }
-            }
-        }
-        if (kt + 1 < nkt)
-            swrite(buf ^ 1);
-        __syncthreads();
-    }
-
-    const float lt = sum_xor32(l_run);
-    const float inv = (lt > 0.f) ? 1.0f / lt : 0.f;
-    if (myq < Sq) {
-        float *orow = O + ((size_t)h * Sq + myq) * D;
-        // O^T register (db, i) of this lane holds d = 32db + 8(i/4) + 4hi + i%4.
-#pragma unroll
-        for (int db = 0; db < DP / 32; ++db)
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                const int d = db * 32 + i4 * 8 + 4 * hi;
-                f32x4 v = {o[db][4 * i4] * inv, o[db][4 * i4 + 1] * inv, o[db][4 * i4 + 2] * inv,
-                           o[db][4 * i4 + 3] * inv};
-                if (VEC) {
-                    if (d < D)
-                        *reinterpret_cast<f32x4 *>(orow + d) = v;
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (d + j < D)
-                            orow[d + j] = v[j];
-                }
-            }
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// Prefill, fast path: D % 8 == 0 with D <= DP (64, 96, 128 or 256) and 16-byte aligned
-// tensors; the head-dim columns D .. DP-1 are zero in the tiles and in Q, and are never stored.
-// The MFMA tiling of attn_prefill_kernel with NW waves per workgroup (8: 256 query rows, two
-// waves per SIMD; 4 on grids too small to fill the GPU, and always at DP = 256, where one wave
-// per SIMD holds O and Q), plus:
+//   * UA = 0 (D % 8 == 0, 16-byte aligned tensors, kv heads below 2 GiB; V^T: Sk % 8 == 0):
 //   * K/V tiles arrive through raw buffer loads whose range is the kv head's Sk*D*2 bytes, so a
 //     key past Sk reads as zero without a branch. The whole byte offset travels in the VGPR
 //     offset (the range-checked one); the scalar offset is always 0. They are LDS-DMA loads
@@ -544,7 +369,20 @@ constexpr int prefill_wg_per_cu(int DP, int KT, int NW) {
 // 64-key tiles. NW = 12 (DP = 64, non-causal, packed rows): 6 * 32 rows per workgroup, waves
 // w and w + 6 on the same rows, three waves per SIMD; one such workgroup per CU holds the
 // rows of one and a half 128-row tiles with no partials to merge.
-template <int DP, int KT, int NW, bool CAUSAL, bool VT, bool KH>
+//
+// UA = 1 (unaligned): tensors without the vector layout (D % 8 != 0, a base that is not 16-byte
+// aligned, V^T rows of an odd key count, or a kv head past a buffer's 31-bit range). The same tiles
+// and LDS layouts, but each 16-byte piece goes through registers: loaded at element alignment at the
+// start of the tile before, put into LDS at its end. What bounds it is those loads (2-byte aligned
+// ones cost 6% more than 4-byte aligned ones, which cost what 16-byte aligned ones do), the registers
+// they hold (two pieces per thread and tensor on 64-key tiles at 8 waves; on 4 waves, or K waited
+// for in mid-tile, 27-75% slower) and the row max, which every tile takes: the largest weights
+// of a row are then exactly 1 or close below (error against 64 bits 1.5e-3 of the result, 1.7e-3
+// with the sum test, which was 8% faster). Same box, element-wise loads before -> now: 24 heads of
+// 1000 rows over 2003 keys, D = 100, V^T with its pack 249 -> 57 us; 64 heads at 2k, D = 128, V^T
+// of 2003 keys 950 -> 172 us; D = 100 causal 524 -> 118 us (aligned, D = 128: 126 us non-causal).
+// UA = 2: rows shorter than a piece (D < 8), read element by element.
+template <int DP, int KT, int NW, bool CAUSAL, bool VT, bool KH, int UA>
 __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_prefill_fast_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     const uint16_t *__restrict__ V, float *__restrict__ O, int Hq, int Hkv, int Sq, int Sk, int D,
@@ -556,6 +394,8 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     static_assert(!KH || (KT == 128 && ((NW == 8 && DP >= 64) || (NW == 12 && DP == 64 && !CAUSAL))),
                   "key halves: 8 waves (or 12 at DP = 64), 128-key tiles");
     static_assert(NW != 12 || KH, "12 waves: key halves only");
+    // Software-pipelined tiles (tile_pipelined): D <= 64, key halves on 12 waves only.
+    constexpr bool kPipe = DP <= 64 && (!KH || NW == 12) && !UA;
     constexpr int NR = KH ? NW / 2 : NW; // waves with distinct query rows
     constexpr int KW = KH ? KT / 2 : KT; // keys of a tile that one wave takes
     constexpr int BQ = NR * 32;         // query rows per workgroup
@@ -693,7 +533,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     // (c3 1k causal, chunked prefill), and they, packed tiles and DP = 256 load directly.
     constexpr int NQC = DP / 8; // 16-byte chunks per Q row
     constexpr int QSWZ = (NQC % 16 == 0) ? 15 : ((NQC % 8 == 0) ? 7 : 3);
-    const bool qstage = NW == 8 && KT >= 16 * NW && DP <= 128 && !pack &&
+    const bool qstage = !UA && NW == 8 && KT >= 16 * NW && DP <= 128 && !pack &&
                         (long)Sq * D * 2 < 0x7fffffffL;
     const uint16_t *qlds =
         NW == 8 ? (w < NW / 2 ? &Ks[1][0] : &Vs[1][0]) + (w % (NW / 2)) * 32 * DP : &Ks[1][0];
@@ -710,7 +550,8 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     } else {
 #pragma unroll
         for (int kk = 0; kk < DP / 16; ++kk)
-            qb[kk] = as_bf16x8(load_row8<true>(Q, qrow, kk * 16 + hi * 8, D, rvalid));
+            qb[kk] = as_bf16x8(load_row8<UA == 0, false, UA == 2>(Q, qrow, kk * 16 + hi * 8, D,
+                                                                  rvalid, kk * 16 + 16));
     }
     // Q stays in flight while the first tile's DMA is issued; one wait before the loop covers
     // both (below).
@@ -793,6 +634,109 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         for (int k = 0; k < PW; ++k)
             if (NI % NW == 0 || k < nblk_w)
                 dma16<0>(rkt, &Ks[buf][(w * PW + k) * 512], kso[k]);
+    };
+    // UA: this wave's pieces of a K (or V) tile into registers, and from there into LDS. Every load
+    // stays inside its row: a piece that reaches past the row's end is read as the row's last
+    // eight elements and shifted where it is put into LDS (shifting it at the load would wait for
+    // it). One packed offset per piece is kept and made opaque where it is used: what follows
+    // from it would otherwise be hoisted out of the key loop and spilled.
+    constexpr int UPW = UA ? PW : 1;
+    constexpr bool TINY = UA == 2; // rows of fewer than eight elements: element by element
+    u32x4 gk[UPW], gv[UPW];
+    const uint16_t *Kh = K + (size_t)u * Sk * D, *Vh = V + (size_t)u * Sk * D;
+    // Row-major piece k: (element offset of its eight elements in the tile) * 16 + how many of
+    // them precede the piece. TINY: (row * 64 + first column).
+    uint32_t kpk[UPW], vpk[UPW];
+    uint32_t ktail = 0, vtail = 0; // bit k: piece k of some lane reaches past D (wave-uniform)
+    if constexpr (UA != 0) {
+        auto pack = [&](int r, int col, uint32_t &pk, uint32_t &tail, int k) {
+            pk = TINY ? (uint32_t)(r * 64 + col)
+                      : (uint32_t)(r * D + min(col, D - 8)) * 16u + (uint32_t)min(8, max(0, col + 8 - D));
+            tail |= __builtin_amdgcn_ballot_w64(col + 8 > D) != 0 ? 1u << k : 0u;
+        };
+#pragma unroll
+        for (int k = 0; k < PW; ++k) {
+            const int b = (w * PW + k) * 1024 + 16 * lane;
+            const int rk = b / (16 * DP), wk = b % (16 * DP), rw = b / (8 * DP), wv = b % (8 * DP);
+            pack(rk * 8 + (wk % 256) / 32, 8 * (2 * (wk / 256) + (((wk % 32) / 16) ^ (rk & 1))),
+                 kpk[k], ktail, k);
+            pack(rw * 4 + (wv % 256) / 64, 8 * (4 * (wv / 256) + (wv % 64) / 16), vpk[k], vtail, k);
+        }
+        ktail = __builtin_amdgcn_readfirstlane(ktail);
+        vtail = __builtin_amdgcn_readfirstlane(vtail);
+    }
+    auto opaque = [](uint32_t x) __attribute__((always_inline)) {
+        asm volatile("" : "+v"(x));
+        return x;
+    };
+    auto ua_rows = [&](const uint16_t *H, int kt, const uint32_t *pk, u32x4 *gr)
+        __attribute__((always_inline)) {
+        const uint16_t *T = H + (size_t)kt * KT * D;
+        const uint32_t last = (uint32_t)((Sk - kt * KT) * (long)D > KT * DP ? KT * DP
+                                                                            : (Sk - kt * KT) * D);
+#pragma unroll
+        for (int k = 0; k < PW; ++k)
+            if (NI % NW == 0 || k < nblk_w) {
+                const uint32_t x = opaque(pk[k]);
+                if constexpr (TINY) {
+                    const int r = (int)(x >> 6), col = (int)(x & 63);
+                    gr[k] = zero4();
+                    if (kt * KT + r < Sk && col < D)
+                        gr[k] = load_run8(T + r * D, col, D, true);
+                } else { // rows past the last key read its last elements
+                    gr[k] = load16_any<false>(T + min(x >> 4, last - 8));
+                }
+            }
+    };
+    // Rows past the last key become zeros (their P is 0, and 0 times what was read may be NaN).
+    auto put_rows = [&](uint16_t *tile, int kt, const uint32_t *pk, uint32_t tail, const u32x4 *gr)
+        __attribute__((always_inline)) {
+        const bool edge = !TINY && kt * KT + KT > Sk;
+#pragma unroll
+        for (int k = 0; k < PW; ++k)
+            if (NI % NW == 0 || k < nblk_w) {
+                u32x4 v = gr[k];
+                if (!TINY && (tail >> k & 1))
+                    v = drop_elems(v, (int)(opaque(pk[k]) & 15));
+                if (edge)
+                    v = (int)(opaque(pk[k]) >> 4) < (Sk - kt * KT) * D ? v : zero4();
+                *reinterpret_cast<u32x4 *>(&tile[(w * PW + k) * 512 + lane * 8]) = v;
+            }
+    };
+    // V^T piece k: d row e (past D: D - 1, never stored) and the eight keys from 8 kc of the tile.
+    auto vt_piece = [&](int k, int &e, int &key) __attribute__((always_inline)) {
+        const int b = (w * PW + k) * 1024 + 16 * (int)opaque((uint32_t)lane);
+        const int rg = b / (16 * KT), wi = b % (16 * KT);
+        e = min(rg * 8 + (wi % 256) / 32, D - 1);
+        key = 8 * (2 * (wi / 256) + (((wi % 32) / 16) ^ (rg & 1)));
+    };
+    auto ua_vt = [&](int kt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < PW; ++k)
+            if (NI % NW == 0 || k < nblk_w) {
+                int e, key;
+                vt_piece(k, e, key);
+                key += kt * KT;
+                const uint16_t *row = Vh + (size_t)e * Sk;
+                if (TINY || Sk < 8)
+                    gv[k] = key < Sk ? load_run8(row, key, Sk, true) : zero4();
+                else
+                    gv[k] = load16_any<false>(row + min(key, Sk - 8));
+            }
+    };
+    auto put_vt = [&](uint16_t *tile, int kt) __attribute__((always_inline)) {
+        const bool edge = !TINY && Sk >= 8 && kt * KT + KT > Sk;
+#pragma unroll
+        for (int k = 0; k < PW; ++k)
+            if (NI % NW == 0 || k < nblk_w) {
+                u32x4 v = gv[k];
+                if (edge) {
+                    int e, key;
+                    vt_piece(k, e, key);
+                    v = drop_elems(v, min(8, max(0, kt * KT + key + 8 - Sk)));
+                }
+                *reinterpret_cast<u32x4 *>(&tile[(w * PW + k) * 512 + lane * 8]) = v;
+            }
     };
     auto dma_v = [&](int kt, int buf) {
         if constexpr (VT) {
@@ -1121,9 +1065,33 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
             }
     };
 
+    // The staging of tile kt into buffer buf: by DMA at the start of the tile before it, or (UA)
+    // loaded at that tile's start and put into LDS at its end.
+    auto stage_begin = [&](int kt, int buf) __attribute__((always_inline)) {
+        if constexpr (UA != 0) {
+            ua_rows(Kh, kt, kpk, gk);
+            if constexpr (VT)
+                ua_vt(kt);
+            else
+                ua_rows(Vh, kt, vpk, gv);
+        } else {
+            dma_k(kt, buf);
+            dma_v(kt, buf);
+        }
+    };
+    auto stage_end = [&](int kt, int buf) __attribute__((always_inline)) {
+        if constexpr (UA != 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            put_rows(&Ks[buf][0], kt, kpk, ktail, gk);
+            if constexpr (VT)
+                put_vt(&Vs[buf][0], kt);
+            else
+                put_rows(&Vs[buf][0], kt, vpk, vtail, gv);
+        }
+    };
     if (kt0 < kt1) {
-        dma_k(kt0, 0);
-        dma_v(kt0, 0);
+        stage_begin(kt0, 0);
+        stage_end(kt0, 0);
     }
     // Q and this wave's DMA blocks of the first tile have landed. Q must be resident before the
     // loop: otherwise the compiler's wait at the loop's first MFMA also waits for the next tile's
@@ -1143,10 +1111,8 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     auto step = [&](int kt, auto first, auto me) __attribute__((always_inline)) {
         const int buf = (kt - kt0) & 1;
         // The other buffer's last readers finished before the barrier that ended tile kt-1.
-        if (kt + 1 < kt1) {
-            dma_k(kt + 1, buf ^ 1);
-            dma_v(kt + 1, buf ^ 1);
-        }
+        if (kt + 1 < kt1)
+            stage_begin(kt + 1, buf ^ 1);
         const int kbase = kt * KT + kh * KW; // this wave's keys: [kbase, kbase + KW)
         const bool edge = decltype(me)::value &&
                           ((kbase + KW > Sk) || (CAUSAL && kbase + KW - 1 > Sk - Sq + qmin));
@@ -1154,13 +1120,13 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
             // The pipelined path at DP <= 64 only: at larger DP it spills (two sub-tiles' K
             // fragments, S and the V read-ahead do not fit beside O and Q). Key halves take it
             // on 12 waves only (two 32-key sub-tiles per wave).
-            if (DP <= 64 && (!KH || NW == 12) && !decltype(first)::value && !edge && pipe) {
-                if constexpr (DP <= 64 && (!KH || NW == 12))
+            if (kPipe && !decltype(first)::value && !edge && pipe) {
+                if constexpr (kPipe)
                     tile_pipelined(buf);
             } else {
                 qk(buf);
                 pv_first(buf);
-                if constexpr (decltype(first)::value) {
+                if constexpr (UA || decltype(first)::value) {
                     mask(kbase, me);
                     row_max();
                     l_run += exps();
@@ -1174,6 +1140,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         // buffer buf for tile kt+2. After the item's last tile there is neither: its epilogue
         // uses only the idle buffer (below), so each wave goes on without waiting for the others.
         if (kt + 1 < kt1) {
+            stage_end(kt + 1, buf ^ 1);
             __builtin_amdgcn_s_waitcnt(0x0F70);
             __syncthreads();
         }
@@ -1196,7 +1163,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
             step(kt, std::false_type{}, std::true_type{});
     } else {
         int kt = kt0 + 1;
-        if constexpr (DP <= 64 && (!KH || NW == 12)) {
+        if constexpr (kPipe) {
             // A wave with query rows runs its tiles before kt_e (no mask needed) in a loop of
             // their own whose body is the pipelined tile alone: with the general tile path in
             // the same loop body, the register allocator kept o in different registers on the
@@ -1209,10 +1176,8 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
             if (pipe && __builtin_amdgcn_readfirstlane(wave_maxkey) >= 0) {
                 for (; kt < min(kt1, kt_e); ++kt) {
                     const int buf = (kt - kt0) & 1;
-                    if (kt + 1 < kt1) {
-                        dma_k(kt + 1, buf ^ 1);
-                        dma_v(kt + 1, buf ^ 1);
-                    }
+                    if (kt + 1 < kt1)
+                        stage_begin(kt + 1, buf ^ 1);
                     tile_pipelined(buf);
                     // The same wait and barrier as the end of step().
                     if (kt + 1 < kt1) {
@@ -1274,6 +1239,20 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     }
     phase_stamp(w, lane, 4);
     const float lt = sum_xor32(l_run);
+    // Columns d .. d+3 of a row of D floats: UA rows are 4-byte aligned and may end inside them.
+    auto store4 = [&](float *row, int d, f32x4 v) __attribute__((always_inline)) {
+        if constexpr (!UA) {
+            if (d < D)
+                *reinterpret_cast<f32x4 *>(row + d) = v;
+        } else if (d + 4 <= D) {
+            *reinterpret_cast<f32x4_a4 *>(row + d) = v;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (d + j < D)
+                    row[d + j] = v[j];
+        }
+    };
     if (part >= 0 || nsplit > 1) {
         // Unnormalised partial of one key range: (m, l, acc) into slot (row, part) for the
         // log-sum-exp merge (attn_merge2_kernel / attn_merge_kernel).
@@ -1293,8 +1272,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
                 for (int i4 = 0; i4 < 4; ++i4) {
                     const int d = db * 32 + i4 * 8 + 4 * hi;
                     f32x4 v = {o[db][4 * i4], o[db][4 * i4 + 1], o[db][4 * i4 + 2], o[db][4 * i4 + 3]};
-                    if (d < D)
-                        *reinterpret_cast<f32x4 *>(prow + d) = v;
+                    store4(prow, d, v);
                 }
         }
 #if ATTN_PHASE_STAMPS
@@ -1359,8 +1337,8 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
                     const int f = q * 64 + lane, r = f / NCP, c = f - r * NCP;
                     const f32x4 v =
                         *reinterpret_cast<const f32x4 *>(ob + r * (NCP * 4) + ((c ^ key(r)) * 4));
-                    if (row0 + r < Sq && col0 + c * 4 < D)
-                        *reinterpret_cast<f32x4 *>(obase + (size_t)r * D + col0 + c * 4) = v;
+                    if (row0 + r < Sq)
+                        store4(obase + (size_t)r * D, col0 + c * 4, v);
                 }
             }
         }
@@ -1374,8 +1352,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
                 const int d = db * 32 + i4 * 8 + 4 * hi;
                 f32x4 v = {o[db][4 * i4] * inv, o[db][4 * i4 + 1] * inv, o[db][4 * i4 + 2] * inv,
                            o[db][4 * i4 + 3] * inv};
-                if (d < D)
-                    *reinterpret_cast<f32x4 *>(orow + d) = v;
+                store4(orow, d, v);
             }
     }
 #if ATTN_PHASE_STAMPS
@@ -2125,7 +2102,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 #pragma unroll
     for (int kk = 0; kk < DP / 32; ++kk)
         qb[kk] = as_bf16x8(
-            load_row8<VEC>(Q + (size_t)h * Sq * D, (size_t)qi, kk * 32 + grp * 8, D, rvalid));
+            load_row8<VEC>(Q + (size_t)h * Sq * D, (size_t)qi, kk * 32 + grp * 8, D, rvalid,
+                           kk * 32 + 32));
     const int lim = CAUSAL ? min(Sk - 1, Sk - Sq + qi) : Sk - 1;
 
     float m_run = kNegInf, l_run = 0.f;
@@ -2151,14 +2129,15 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
             const int key = tb + 8 * (r16 >> 2) + 4 * t + (r16 & 3);
 #pragma unroll
             for (int kk = 0; kk < DP / 32; ++kk)
-                ka[t][kk] = load_row8<VEC, NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1);
+                ka[t][kk] = load_row8<VEC, NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1,
+                                                kk * 32 + 32);
         }
         u32x4 vv[VT ? DP / 16 : VNCH];
         if (VT) {
             // lane: d row 16db + r16, keys tb + 8grp .. +7 (the k index of pk below).
 #pragma unroll
             for (int db = 0; db < DP / 16; ++db)
-                vv[db] = load_vt8<VEC, NTL>(Vh, db * 16 + r16, tb + 8 * grp, Sk, D, k1);
+                vv[db] = load_vt8<VEC, NTL>(Vh, db * 16 + r16, tb + 8 * grp, Sk, D, k1, tb + 32);
         } else {
 #pragma unroll
             for (int r = 0; r < VNCH; ++r) {
@@ -2292,7 +2271,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 // kernels' outputs are bit-identical. The 16-byte chunks of a tile row e sit at slot
 // c ^ (e % 16), so the 16 lanes of an operand read (16 d rows, one key chunk) hit 16 distinct
 // bank groups. NTL: K loads and V^T DMA are non-temporal (decode_nt_loads decides).
-template <int DP, bool CAUSAL, bool NTL>
+template <int DP, bool CAUSAL, bool NTL, bool UA>
 __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     const uint16_t *__restrict__ V, float *__restrict__ O, float *__restrict__ pm,
@@ -2329,7 +2308,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
 #pragma unroll
     for (int kk = 0; kk < DP / 32; ++kk)
         qb[kk] = as_bf16x8(
-            load_row8<true>(Q + (size_t)h * Sq * D, (size_t)qi, kk * 32 + grp * 8, D, rvalid));
+            load_row8<!UA>(Q + (size_t)h * Sq * D, (size_t)qi, kk * 32 + grp * 8, D, rvalid,
+                           kk * 32 + 32));
     const int lim = CAUSAL ? min(Sk - 1, Sk - Sq + qi) : Sk - 1;
 
     float m_run = kNegInf, l_run = 0.f;
@@ -2342,7 +2322,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
     // tile row e receives source chunk p ^ (e % 16) (tiles start at multiples of 16 d rows, so
     // e % 16 is also the d row's). A chunk of a d row past D or of keys at or past k1 gets an
     // offset beyond the buffer's range and lands as zeros.
-    const __amdgpu_buffer_rsrc_t rvt = make_rsrc(V + (size_t)u * D * Sk, (uint32_t)D * Sk * 2);
+    const uint16_t *Vh = V + (size_t)u * D * Sk;
+    const __amdgpu_buffer_rsrc_t rvt = make_rsrc(Vh, (uint32_t)D * Sk * 2);
     const uint32_t row_bytes = (uint32_t)Sk * 2u;
     uint32_t vsrc[RPW];
     int vkey[RPW];
@@ -2360,15 +2341,38 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
     const int ngr = (nsteps + 3) / 4;
     const int rot = us % (nsteps > 0 ? nsteps : 1);
     auto step_of = [&](int js) { return (js + rot < nsteps) ? js + rot : js + rot - nsteps; };
+    // UA: the tile's pieces go through registers (vr), loaded where the DMA would be issued and
+    // written at the interval's end (put_tile).
+    u32x4 vr[UA ? RPW : 1];
     auto dma_tile = [&](int j, int q, int buf) {
         const int pos = 4 * j + (lane >> 4); // this lane's walk position
         const int key0 = pos < nsteps ? k0 + step_of(pos) * 128 : k1;
         const int klim = k1 - key0; // keys of this lane's step inside the split
+        if constexpr (UA) {
+            // Every load stays inside its row's first k1 keys (k1 >= 8): a piece that reaches past
+            // k1 reads the last eight and is shifted in put_tile. Rows past D are never stored.
+#pragma unroll
+            for (int k = 0; k < RPW; ++k)
+                vr[k] = load16_any<NTL>(Vh + (size_t)min(q * RQ + w * RPW + k, D - 1) * Sk +
+                                        min(key0 + vkey[k], k1 - 8));
+            return;
+        }
         const uint32_t base = (uint32_t)(q * RQ) * row_bytes + (uint32_t)key0 * 2u;
 #pragma unroll
         for (int k = 0; k < RPW; ++k) {
             const bool ok = q * RQ + w * RPW + k < D && vkey[k] < klim;
             dma16<0, NTL ? kDmaNT : 0>(rvt, &Vt[buf][(w * RPW + k) * GK], ok ? vsrc[k] + base : 0x80000000u);
+        }
+    };
+    auto put_tile = [&](int j, int buf) {
+        const int pos = 4 * j + (lane >> 4);
+        const int key0 = pos < nsteps ? k0 + step_of(pos) * 128 : k1;
+        const bool may = __builtin_amdgcn_ballot_w64(key0 + 128 > k1) != 0;
+#pragma unroll
+        for (int k = 0; k < (UA ? RPW : 0); ++k) {
+            if (may)
+                vr[k] = drop_elems(vr[k], min(8, max(0, key0 + vkey[k] + 8 - k1)));
+            *reinterpret_cast<u32x4 *>(&Vt[buf][(w * RPW + k) * GK + lane * 8]) = vr[k];
         }
     };
     u32x4 ka[2][DP / 32], kn[2][DP / 32];
@@ -2378,7 +2382,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
             const int key = tb + 8 * (r16 >> 2) + 4 * t + (r16 & 3);
 #pragma unroll
             for (int kk = 0; kk < DP / 32; ++kk)
-                dst[t][kk] = load_row8<true, NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1);
+                dst[t][kk] = load_row8<!UA, NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1,
+                                                 kk * 32 + 32);
         }
     };
 
@@ -2476,6 +2481,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
                     for (int kk = 0; kk < DP / 32; ++kk)
                         ka[t][kk] = kn[t][kk];
             }
+            if (UA && (i < 3 ? j > 0 : cur))
+                put_tile(i < 3 ? j - 1 : j, buf ^ 1);
             buf ^= 1;
         });
 #pragma unroll
@@ -2707,36 +2714,15 @@ __global__ __launch_bounds__(256) void attn_merge2_kernel(const float *__restric
     }
 }
 
-// V [Hkv][Sk][D] -> Vp [Hkv][D][Sk] through a 32x32 LDS tile (block 32x8).
-__global__ __launch_bounds__(256) void attn_pack_v_kernel(const uint16_t *__restrict__ V,
-                                                          uint16_t *__restrict__ Vp, int Sk,
-                                                          int D) {
-    __shared__ uint16_t tile[32][33];
-    const int kv = wg_id_z();
-    const int k0 = wg_id_x() * 32, d0 = wg_id_y() * 32;
-    const int tx = wi_id_x(), ty = wi_id_y();
-    const uint16_t *src = V + (size_t)kv * Sk * D;
-    uint16_t *dst = Vp + (size_t)kv * D * Sk;
-    for (int r = ty; r < 32; r += 8) {
-        const int k = k0 + r, d = d0 + tx;
-        tile[r][tx] = (k < Sk && d < D) ? src[(size_t)k * D + d] : (uint16_t)0;
-    }
-    __syncthreads();
-    for (int r = ty; r < 32; r += 8) {
-        const int d = d0 + r, k = k0 + tx;
-        if (d < D && k < Sk)
-            dst[(size_t)d * Sk + k] = tile[tx][r];
-    }
-}
-
-// V [Hkv][Sk][D] -> Vp [Hkv][D][Sk] when D % 8 == 0, Sk % 8 == 0 and both tensors are 16-byte
-// aligned: one workgroup per TK-key x 64-column tile. Key rows arrive as 16-byte loads into LDS;
+// V [Hkv][Sk][D] -> Vp [Hkv][D][Sk]: one workgroup per TK-key x 64-column tile. Key rows arrive as 16-byte loads into LDS;
 // each thread then gathers 8 consecutive keys of one column and stores them as one 16-byte
 // chunk, so each wave store writes 512 / TK columns x 2*TK contiguous bytes.
 // The LDS tile has unpadded 128-byte rows, 16-byte chunk c of row r stored at chunk
 // c ^ ((r >> 3) & 7). The gathers of a wave read one column chunk of TK/8 rows spaced 8 apart;
 // the XOR sends each 8 consecutive such rows to 8 different chunks.
-template <int TK>
+// VEC: D % 8 == 0, Sk % 8 == 0 and both tensors 16-byte aligned. Otherwise the same 16-byte pieces
+// at element alignment, the ends of rows handled apart.
+template <int TK, bool VEC>
 __global__ __launch_bounds__(256) void attn_pack_v16_kernel(const uint16_t *__restrict__ V,
                                                             uint16_t *__restrict__ Vp, int Sk,
                                                             int D) {
@@ -2756,7 +2742,9 @@ __global__ __launch_bounds__(256) void attn_pack_v16_kernel(const uint16_t *__re
         const int k = k0 + row, d = d0 + ch * 8;
         u32x4 v = zero4();
         if (k < Sk && d < D)
-            v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + (size_t)k * D + d));
+            v = VEC ? __builtin_nontemporal_load(
+                          reinterpret_cast<const u32x4 *>(src + (size_t)k * D + d))
+                    : load_run8<true>(src + (size_t)k * D, d, D, d0 + TD > D);
         *reinterpret_cast<u32x4 *>(&tile[row * TD + ((ch ^ (row >> 3)) & 7) * 8]) = v;
     }
     __syncthreads();
@@ -2773,7 +2761,17 @@ __global__ __launch_bounds__(256) void attn_pack_v16_kernel(const uint16_t *__re
                 e[j] = tile[(kc + j) * TD + col];
             const u32x4 out = {e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16),
                                e[6] | (e[7] << 16)};
-            *reinterpret_cast<u32x4 *>(dst + (size_t)d * Sk + k) = out;
+            uint16_t *q = dst + (size_t)d * Sk + k;
+            if (VEC) {
+                *reinterpret_cast<u32x4 *>(q) = out;
+            } else if (k + 8 <= Sk) {
+                *reinterpret_cast<u32x4_a2 *>(q) = out;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 7; ++j)
+                    if (k + j < Sk)
+                        q[j] = (uint16_t)e[j];
+            }
         }
     }
 }
@@ -2817,22 +2815,6 @@ __attribute__((format(printf, 3, 4))) void plan_note(dim3 g, dim3 b, const char 
     memcpy(p->buf + p->pos, line, used);
     p->pos += used;
     p->buf[p->pos] = '\0';
-}
-
-template <int DP, int KT, bool CAUSAL, bool VEC, bool VT>
-hipError_t launch_prefill_t(const uint16_t *Q, const uint16_t *K, const uint16_t *V, float *O,
-                            int Hq, int Hkv, int Sq, int Sk, int D, float c, hipStream_t st) {
-    const int nqt = (Sq + 127) / 128;
-    const long nblk = (long)Hq * nqt;
-    if (nblk <= 0 || nblk > 0x7fffffffL)
-        return hipErrorInvalidValue;
-    if (t_plan)
-        plan_note(dim3((unsigned)nblk), dim3(256), "attn_prefill_kernel<%d, %d, %s, %s, %s>", DP,
-                  KT, tf(CAUSAL), tf(VEC), tf(VT));
-    else
-        hipLaunchKernelGGL((attn_prefill_kernel<DP, KT, CAUSAL, VEC, VT>), dim3((unsigned)nblk),
-                           dim3(256), 0, st, Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, nqt);
-    return hipGetLastError();
 }
 
 hipError_t launch_merge(const float *pm, const float *pl, const float *pacc, float *O, long rows,
@@ -2995,7 +2977,7 @@ static bool prefill_rows192(int Hq, int Hkv, int Sq) {
 // A causal grid of at most one workgroup per CU is as slow as its heaviest query tile. Then the
 // key range of each tile in the upper half (qt >= nqt/2) is split in two workgroups whose
 // partials (m, l, acc) go to the caller's scratch and are merged, when the slots suffice.
-template <int DP, int KT, int NW, bool CAUSAL, bool VT, bool KH = false>
+template <int DP, int KT, int NW, bool CAUSAL, bool VT, bool KH = false, int UA = 0>
 hipError_t launch_prefill_fast_nw(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                   float *O, int Hq, int Hkv, int Sq, int Sk, int D, float c,
                                   float *pm, float *pl, float *pacc, long slots, hipStream_t st) {
@@ -3048,12 +3030,12 @@ hipError_t launch_prefill_fast_nw(const uint16_t *Q, const uint16_t *K, const ui
                                                    nblk);
     if (t_plan)
         plan_note(dim3((unsigned)nblk), dim3(NW * 64),
-                  "attn_prefill_fast_kernel<%d, %d, %d, %s, %s, %s> nsplit=%d split_first=%d "
+                  "attn_prefill_fast_kernel<%d, %d, %d, %s, %s, %s%s> nsplit=%d split_first=%d "
                   "hsplit=%d pack=%d pair=%d",
-                  DP, KT, NW, tf(CAUSAL), tf(VT), tf(KH), nsplit, split_first, hsplit, pack,
-                  pair_r);
+                  DP, KT, NW, tf(CAUSAL), tf(VT), tf(KH), UA ? ", unaligned" : "", nsplit,
+                  split_first, hsplit, pack, pair_r);
     else
-        hipLaunchKernelGGL((attn_prefill_fast_kernel<DP, KT, NW, CAUSAL, VT, KH>),
+        hipLaunchKernelGGL((attn_prefill_fast_kernel<DP, KT, NW, CAUSAL, VT, KH, UA>),
                            dim3((unsigned)nblk), dim3(NW * 64), 0, st, Q, K, V, O, Hq, Hkv, Sq, Sk,
                            D, c, nqt, split_first, pm, pl, pacc, prows, pack, pair_r,
                            prefill_pipe(), nsplit, (int)nblk, hsplit);
@@ -3291,33 +3273,54 @@ hipError_t launch_prefill_fast_t(const uint16_t *Q, const uint16_t *K, const uin
                                                           pl, pacc, slots, st);
 }
 
-// The fast kernel needs D % 8 == 0 with D <= DP, 16-byte vectors (vec; with V^T also
+// Unaligned tensors (UA): the aligned kernels' choice of workgroup, without the persistent, head
+// split and 12-wave variants, on 64-key tiles (two staged pieces per thread and tensor at 8 waves).
+template <int DP, int KT, bool CAUSAL, bool VT>
+hipError_t launch_prefill_ua(const uint16_t *Q, const uint16_t *K, const uint16_t *V, float *O,
+                             int Hq, int Hkv, int Sq, int Sk, int D, float c, float *pm, float *pl,
+                             float *pacc, long slots, hipStream_t st) {
+    constexpr int KT4 = (DP > 128) ? 32 : (DP > 64 && KT == 128) ? 64 : KT;
+    if constexpr (DP == 64)
+        if (D < 8)
+            return launch_prefill_fast_nw<DP, KT4, 4, CAUSAL, VT, false, 2>(
+                Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm, pl, pacc, slots, st);
+    if constexpr (DP <= 128) {
+        const int nw = prefill_waves(Hq, Hkv, Sq, Sk, CAUSAL, false);
+        if (nw == 4 && !prefill_pack(Hq, Hkv, Sq) && prefill_kh(DP, Hq, Sq, Sk, CAUSAL))
+            return launch_prefill_fast_nw<DP, KT, 8, CAUSAL, VT, true, 1>(
+                Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm, pl, pacc, slots, st);
+        if (nw == 8)
+            return launch_prefill_fast_nw<DP, KT4, 8, CAUSAL, VT, false, 1>(
+                Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm, pl, pacc, slots, st);
+    }
+    return launch_prefill_fast_nw<DP, KT4, 4, CAUSAL, VT, false, 1>(
+        Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm, pl, pacc, slots, st);
+}
+
+// DMA staging needs D % 8 == 0 with D <= DP, 16-byte vectors (vec; with V^T also
 // Sk % 8 == 0, which the host folds into vec) and a kv head's bytes within a buffer's 31-bit
-// range. D in (64, 96] takes the 96-wide instance, whose MFMA tiles waste less on padding.
-// The general kernel keeps a 64-key tile at DP = 128: its 4-wave tiling at 128 keys would need
-// all 256 registers and drop to one wave per SIMD.
+// range; other calls take the unaligned instances. D in (64, 96] takes the 96-wide instance,
+// whose MFMA tiles waste less on padding.
 template <int DP, int KT>
 hipError_t launch_prefill_dk(const uint16_t *Q, const uint16_t *K, const uint16_t *V, float *O,
                              int Hq, int Hkv, int Sq, int Sk, int D, int causal, int vec, int vt,
                              float c, float *pm, float *pl, float *pacc, long slots,
                              hipStream_t st) {
-    constexpr int KTG = (DP == 256) ? 32 : ((DP == 128 && KT == 128) ? 64 : KT);
     const bool fast = vec && D % 8 == 0 && D <= DP && (long)Sk * D * 2 < 0x7fffffffL;
     return with_flag(causal != 0, [&](auto CA) {
         return with_flag(vt != 0, [&](auto VTF) {
             constexpr bool kC = decltype(CA)::value, kT = decltype(VTF)::value;
-            if (fast) {
-                if constexpr (DP == 128)
-                    if (D <= 96)
-                        return launch_prefill_fast_t<96, KT, kC, kT>(Q, K, V, O, Hq, Hkv, Sq, Sk, D,
-                                                                     c, pm, pl, pacc, slots, st);
-                return launch_prefill_fast_t<DP, KT, kC, kT>(Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm,
-                                                             pl, pacc, slots, st);
-            }
-            return with_flag(vec != 0, [&](auto VE) {
-                return launch_prefill_t<DP, KTG, kC, decltype(VE)::value, kT>(Q, K, V, O, Hq, Hkv,
-                                                                               Sq, Sk, D, c, st);
-            });
+            auto go = [&](auto DPW) {
+                constexpr int W = decltype(DPW)::value;
+                return fast ? launch_prefill_fast_t<W, KT, kC, kT>(Q, K, V, O, Hq, Hkv, Sq, Sk, D,
+                                                                   c, pm, pl, pacc, slots, st)
+                            : launch_prefill_ua<W, KT, kC, kT>(Q, K, V, O, Hq, Hkv, Sq, Sk, D, c,
+                                                               pm, pl, pacc, slots, st);
+            };
+            if constexpr (DP == 128)
+                if (D <= 96)
+                    return go(std::integral_constant<int, 96>{});
+            return go(std::integral_constant<int, DP>{});
         });
     });
 }
@@ -3328,9 +3331,7 @@ hipError_t launch_prefill_d(const uint16_t *Q, const uint16_t *K, const uint16_t
                             float c, float *pm, float *pl, float *pacc, long slots,
                             hipStream_t st) {
     // Key tiles of 128 keys up to D = 128, the largest that keeps two waves per SIMD. D in
-    // (128, 256]: 64 keys (the fast kernel's two 64-key K and V tiles fill 128 KB of LDS); the
-    // general kernel there takes 32-key tiles, since its staging registers and the 256-wide O
-    // accumulator leave no room for more.
+    // (128, 256]: 64 keys (two 64-key K and V tiles fill 128 KB of LDS).
     return launch_prefill_dk<DP, DP == 256 ? 64 : 128>(Q, K, V, O, Hq, Hkv, Sq, Sk, D, causal, vec,
                                                        vt, c, pm, pl, pacc, slots, st);
 }
@@ -3374,19 +3375,23 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
     const bool ntl = decode_nt_loads(nrb, kps);
     // The staged V^T kernel's DMA offsets are 32-bit: a head's V^T must stay below 2 GiB.
     if constexpr (DP <= 128)
-        if (vt && vec && decode_vt_staged() && (long)D * Sk * 2 < 0x7fffffffL)
+        if (vt && decode_vt_staged() && (vec ? (long)D * Sk * 2 < 0x7fffffffL : Sk >= 8))
             return with_flag(causal != 0, [&](auto CA) {
                 return with_flag(ntl, [&](auto NT) {
-                    if (t_plan)
-                        plan_note(dim3((unsigned)nblk), dim3(256),
-                                  "attn_decode_vt_kernel<%d, %s, %s> nsplit=%d nrb=%d", DP,
-                                  tf(decltype(CA)::value), tf(decltype(NT)::value), nsplit, nrb);
-                    else
-                        hipLaunchKernelGGL(
-                            (attn_decode_vt_kernel<DP, decltype(CA)::value, decltype(NT)::value>),
-                            dim3((unsigned)nblk), dim3(256), 0, st, Q, K, V, O, pm, pl, pacc, Hq,
-                            Hkv, Sq, Sk, D, c, nsplit, kps, nrb);
-                    return hipGetLastError();
+                    return with_flag(vec == 0, [&](auto UAF) {
+                        constexpr bool kC = decltype(CA)::value, kN = decltype(NT)::value,
+                                       kU = decltype(UAF)::value;
+                        if (t_plan)
+                            plan_note(dim3((unsigned)nblk), dim3(256),
+                                      "attn_decode_vt_kernel<%d, %s, %s%s> nsplit=%d nrb=%d", DP,
+                                      tf(kC), tf(kN), kU ? ", unaligned" : "", nsplit, nrb);
+                        else
+                            hipLaunchKernelGGL((attn_decode_vt_kernel<DP, kC, kN, kU>),
+                                               dim3((unsigned)nblk), dim3(256), 0, st, Q, K, V, O,
+                                               pm, pl, pacc, Hq, Hkv, Sq, Sk, D, c, nsplit, kps,
+                                               nrb);
+                        return hipGetLastError();
+                    });
                 });
             });
     return with_flag(causal != 0, [&](auto CA) {
@@ -3506,7 +3511,9 @@ extern "C" int attn_hip_launch_merge(const float *pm, const float *pl, const flo
 
 // Keys per pack tile: 128 (256-byte pieces of each V^T row per store). Measured on c3 4k V
 // (inputs rotated past the Infinity Cache): 64 keys 14.1 us, 128 keys 12.65 us, 256 keys 14.4 us,
-// 512 keys 17.8 us.
+// 512 keys 17.8 us. Without the vector layout the same tiles read and write 16 bytes at element
+// alignment; against 32 x 32 tiles of
+// single elements, packing 6 heads of 2003 keys at D = 100 and attending 59.1 -> 56.8 us.
 constexpr int kPackTK = 128;
 
 extern "C" int attn_hip_launch_pack_v(const uint16_t *V, uint16_t *Vp, int Hkv, int Sk, int D,
@@ -3520,16 +3527,14 @@ extern "C" int attn_hip_launch_pack_v(const uint16_t *V, uint16_t *Vp, int Hkv, 
     for (int h0 = 0; h0 < Hkv; h0 += kMaxZ) {
         const unsigned nh = (unsigned)min(kMaxZ, Hkv - h0);
         const size_t off = (size_t)h0 * Sk * D;
-        if (v16) {
-            constexpr int TK = kPackTK;
-            dim3 grid((unsigned)((Sk + TK - 1) / TK), (unsigned)((D + 63) / 64), nh);
-            hipLaunchKernelGGL(attn_pack_v16_kernel<TK>, grid, dim3(256), 0,
+        constexpr int TK = kPackTK;
+        dim3 grid((unsigned)((Sk + TK - 1) / TK), (unsigned)((D + 63) / 64), nh);
+        if (v16)
+            hipLaunchKernelGGL((attn_pack_v16_kernel<TK, true>), grid, dim3(256), 0,
                                (hipStream_t)stream, V + off, Vp + off, Sk, D);
-        } else {
-            dim3 grid((unsigned)((Sk + 31) / 32), (unsigned)((D + 31) / 32), nh);
-            hipLaunchKernelGGL(attn_pack_v_kernel, grid, dim3(32, 8), 0, (hipStream_t)stream,
-                               V + off, Vp + off, Sk, D);
-        }
+        else
+            hipLaunchKernelGGL((attn_pack_v16_kernel<TK, false>), grid, dim3(256), 0,
+                               (hipStream_t)stream, V + off, Vp + off, Sk, D);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess)
             return (int)e;
