@@ -98,3 +98,27 @@ def test_unaligned_pack(Hkv, Sk, D):
     assert np.all(raw[:PAD + 3] == 0xFFFF) and np.all(raw[PAD + 3 + V.size:] == 0xFFFF)
     src.free()
     dst.free()
+
+
+@pytest.mark.parametrize("case", [
+    # Hq, Hkv, Sq, Sk, D, causal: 192-wide tiles (D in (128, 192]) and the last of the 256-wide
+    (8, 2, 300, 640, 136, 0), (8, 2, 300, 640, 192, 1), (8, 2, 300, 640, 200, 1),
+    (6, 3, 129, 65, 160, 0), (16, 4, 40, 129, 184, 1),
+])
+def test_wide_head_dims(oracle, case):
+    """The wide tiles' loop without a rescale, and its way out: keys whose scores jump from tile to
+    tile (up to 2^9 against a stale maximum of the row) fail the sum test in the middle of it."""
+    Hq, Hkv, Sq, Sk, D, causal = case
+    print("case", case, flush=True)
+    Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, 4242 + D)
+    K = K.reshape(Hkv, Sk, D).copy()
+    K[:, 70::97] = (oracle.f32_to_bf16((oracle.bf16_to_f32(K[:, 70::97].ravel()) * 16))).reshape(
+        K[:, 70::97].shape)
+    rows = oracle.ref_rowset(Sq, 16)
+    R = oracle.attn_ref(Q, K.ravel(), V, Hq, Hkv, Sq, Sk, D, causal, rows, nthreads=8)
+    for vt in (0, 1):
+        Vin = np.ascontiguousarray(V.reshape(Hkv, Sk, D).transpose(0, 2, 1)).ravel() if vt else V
+        O = attend(Q, K.ravel(), Vin, Hq, Hkv, Sq, Sk, D, causal, vt, 0)
+        ok, mad, maxref, nbad = oracle.cmp_rows(R, O, Hq, Sq, D, rows)
+        print("   vt=%d err/scale=%.2e nbad=%d" % (vt, mad / maxref, nbad), flush=True)
+        assert ok and nbad == 0, (case, vt, mad, maxref)

@@ -13,7 +13,7 @@
 //
 // Kernels:
 //   attn_prefill_fast_kernel<DP,KT,NW,CAUSAL,VT,KH,UA>  MFMA prefill, D <= DP in {64, 96, 128,
-//                                          256}; one workgroup = NW waves x 32 rows, or (KH) 8
+//                                          192, 256}; one workgroup = NW waves x 32 rows, or (KH) 8
 //                                          waves over 128 rows on key-tile halves; UA: tensors
 //                                          without the 16-byte vector layout
 //   attn_prefill_persist_kernel<DP,CAUSAL,KH> the same tile code at D <= 128, one 8-wave
@@ -245,9 +245,9 @@ __device__ __forceinline__ void lds_wave_fence() {
 }
 
 // ------------------------------------------------------------------------------------------
-// Prefill, D <= DP (64, 96, 128 or 256); the head-dim columns D .. DP-1 are zero in the tiles and
+// Prefill, D <= DP (64, 96, 128, 192 or 256); the head-dim columns D .. DP-1 are zero in the tiles and
 // in Q, and are never stored. NW waves per workgroup (8: 256 query rows, two waves per SIMD; 4 on
-// grids too small to fill the GPU, and always at DP = 256, where one wave per SIMD holds O and Q);
+// grids too small to fill the GPU, and always past DP = 128, where one wave per SIMD holds O and Q);
 // wave w owns 32 query rows. Per key tile of KT keys (one online-softmax update per tile):
 //   S^T[key][q] = K_tile . Q^T     (v_mfma_f32_32x32x16_bf16, A = K rows from LDS, B = Q regs)
 //   each lane holds one query (q = lane%32) and 16 keys per 32-key sub-tile, so the row max is
@@ -1148,7 +1148,55 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     if (kt0 < kt1)
         step(kt0, std::true_type{}, std::true_type{});
     phase_stamp(w, lane, 2);
-    if constexpr (NW == 4 && DP > 64) {
+    if constexpr (DP > 128 && !UA) {
+        // Unmasked tiles in a loop with no rescale of O in it: with 512 registers O lives in
+        // accumulation registers, and a rescale path in the loop had the register allocator copy
+        // all of O out of them on every tile (128 v_accvgpr_read per 64-key tile at DP = 256). A
+        // tile whose sum test fails leaves the loop, takes the row max outside and comes back.
+        // Bit-identical; same box, 64 heads at 2k: D = 256 323 -> 295 us (933 TFLOP/s), causal
+        // 194 -> 179. One wave per SIMD bounds it: its softmax, LDS reads and MFMAs take turns
+        // (MFMA busy 35% of the clocks). Software-pipelined sub-tiles (8 or 12 fragments ahead)
+        // measured 10% slower than these plain phases, alternating the two Q.K^T accumulators
+        // within 1%.
+        const int medge = CAUSAL ? min(Sk - KT, Sk - Sq + qmin - KT + 1) : Sk - KT;
+        const int kt_e = __builtin_amdgcn_readfirstlane(medge < 0 ? 0 : medge / KT + 1);
+        const int kt_m = __builtin_amdgcn_readfirstlane(wave_maxkey < 0 ? 0 : min(kt1, kt_e));
+        auto finish = [&](int kt, int buf) __attribute__((always_inline)) {
+            pv(buf);
+            if (kt + 1 < kt1) {
+                __builtin_amdgcn_s_waitcnt(0x0F70);
+                __syncthreads();
+            }
+        };
+        int kt = kt0 + 1;
+        for (;;) {
+            bool redo = false;
+            for (; kt < kt_m; ++kt) {
+                const int buf = (kt - kt0) & 1;
+                if (kt + 1 < kt1)
+                    stage_begin(kt + 1, buf ^ 1);
+                qk(buf);
+                pv_first(buf);
+                const float psum = exps();
+                redo = __builtin_amdgcn_ballot_w64(!(psum <= kSumCap)) != 0;
+                if (__builtin_expect(redo, 0))
+                    break;
+                l_run += psum;
+                finish(kt, buf);
+            }
+            if (!redo)
+                break;
+            const int buf = (kt - kt0) & 1;
+            qk(buf);
+            pv_first(buf);
+            row_max();
+            l_run += exps();
+            finish(kt, buf);
+            ++kt;
+        }
+        for (; kt < kt1; ++kt)
+            step(kt, std::false_type{}, std::true_type{});
+    } else if constexpr (NW == 4 && DP > 64) {
         // Tiles from kt_e on may need the mask (keys past Sk, or past the causal limit of the
         // wave's first row); the loop before them has no mask code. Measured (same box) on the
         // 4-wave 64-key-tile kernels: c3 1k causal +3.3%, Qwen3 4k causal +2.8%, 32 heads 2k
@@ -3299,8 +3347,9 @@ hipError_t launch_prefill_ua(const uint16_t *Q, const uint16_t *K, const uint16_
 
 // DMA staging needs D % 8 == 0 with D <= DP, 16-byte vectors (vec; with V^T also
 // Sk % 8 == 0, which the host folds into vec) and a kv head's bytes within a buffer's 31-bit
-// range; other calls take the unaligned instances. D in (64, 96] takes the 96-wide instance,
-// whose MFMA tiles waste less on padding.
+// range; other calls take the unaligned instances. D in (64, 96] takes the 96-wide instance and
+// D in (128, 192] the 192-wide one, whose MFMA tiles waste less on padding (64 heads at 2k, D = 192
+// in 256-wide tiles 294 us, in 192-wide ones 222; D = 160 causal 164 -> 121).
 template <int DP, int KT>
 hipError_t launch_prefill_dk(const uint16_t *Q, const uint16_t *K, const uint16_t *V, float *O,
                              int Hq, int Hkv, int Sq, int Sk, int D, int causal, int vec, int vt,
@@ -3320,6 +3369,9 @@ hipError_t launch_prefill_dk(const uint16_t *Q, const uint16_t *K, const uint16_
             if constexpr (DP == 128)
                 if (D <= 96)
                     return go(std::integral_constant<int, 96>{});
+            if constexpr (DP == 256)
+                if (D <= 192)
+                    return go(std::integral_constant<int, 192>{});
             return go(std::integral_constant<int, DP>{});
         });
     });
