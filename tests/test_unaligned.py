@@ -122,3 +122,29 @@ def test_wide_head_dims(oracle, case):
         ok, mad, maxref, nbad = oracle.cmp_rows(R, O, Hq, Sq, D, rows)
         print("   vt=%d err/scale=%.2e nbad=%d" % (vt, mad / maxref, nbad), flush=True)
         assert ok and nbad == 0, (case, vt, mad, maxref)
+
+
+@pytest.mark.parametrize("case", [
+    # Hq, Hkv, Sq, Sk, D, causal: decode with two 16-row blocks per workgroup and its limits
+    (256, 32, 8, 517, 128, 1),   # four blocks, a five-key last tile
+    (192, 64, 12, 400, 96, 1),   # three blocks, the last of 4 rows
+    (192, 64, 12, 401, 97, 0),   # unaligned
+    (64, 1, 1, 16500, 40, 0),    # one kv head: the cap of 64 splits
+    (64, 16, 16, 1024, 64, 1),
+    # merges: splits of 3 to 64, column counts that end inside a 4-float piece
+    (2, 2, 1, 300, 7, 0), (5, 1, 1, 1500, 101, 0), (8, 8, 1, 4100, 256, 0), (1, 1, 1, 8192, 250, 0),
+    (3, 1, 4, 1030, 66, 1), (512, 128, 4, 1000, 128, 1),
+])
+def test_decode_groups_and_merges(oracle, case):
+    Hq, Hkv, Sq, Sk, D, causal = case
+    print("case", case, ts.attn_flash_plan(Hq, Hkv, Sq, Sk, D, causal), flush=True)
+    Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, 777 + D)
+    Vt = np.ascontiguousarray(V.reshape(Hkv, Sk, D).transpose(0, 2, 1)).ravel()
+    rows = oracle.ref_rowset(Sq, 16)
+    R = oracle.attn_ref(Q, K, V, Hq, Hkv, Sq, Sk, D, causal, rows, nthreads=8)
+    O = attend(Q, K, V, Hq, Hkv, Sq, Sk, D, causal, 0, 0)
+    ok, mad, maxref, nbad = oracle.cmp_rows(R, O, Hq, Sq, D, rows)
+    print("   err/scale=%.2e nbad=%d" % (mad / maxref, nbad), flush=True)
+    assert ok and nbad == 0, (case, mad, maxref)
+    # the same order of sums from V^T, whichever kernel reads it
+    assert np.array_equal(O, attend(Q, K, Vt, Hq, Hkv, Sq, Sk, D, causal, 1, 0)), case

@@ -9,6 +9,8 @@
 #define __HIP_PLATFORM_AMD__ 1
 #include "attn_flash.h"
 
+#include "attn_decode_rule.h"
+
 #include <hip/hip_runtime_api.h>
 #include <math.h>
 #include <stdint.h>
@@ -154,14 +156,20 @@ static int attn_use_decode(int Hkv, int group, int Sq) {
         return 1;
     return rows <= ATTN_DECODE_MAX_ROWS && Hkv < attn_hip_device_cus();
 }
-#define ATTN_DECODE_TARGET_WG 512
-#define ATTN_DECODE_MIN_KEYS 128 /* keys per split: one 32-key tile per wave, 4 waves */
 
-static void attn_decode_split(int Hq, int Hkv, int Sq, int Sk, int nrb, int *nsplit_o,
+static void attn_decode_split(int Hq, int Hkv, int Sq, int Sk, int nrb, int dp, int *nsplit_o,
                               int *kps_o) {
     long rows = (long)Hq * Sq;
     long cap = ATTN_SLOTS / (rows > 0 ? rows : 1);
-    long want = (ATTN_DECODE_TARGET_WG + (long)Hkv * nrb - 1) / ((long)Hkv * nrb);
+    /* Up to D = 128 one workgroup serves the row blocks of a key range, two of them or (at half
+     * the workgroups, one wave per SIMD) four. */
+    /* One workgroup per (kv head, split, group of row blocks). */
+    const int per = attn_decode_blocks(nrb, dp, Hkv, Sk);
+    const long wgs = (long)Hkv * ((nrb + per - 1) / per);
+    long want = (ATTN_DECODE_TARGET_WG + wgs - 1) / wgs;
+    /* Grouped blocks: no more than the 64 splits that one merge wave covers. */
+    if (per > 1 && want > 64)
+        want = 64;
     long by_len = (Sk + ATTN_DECODE_MIN_KEYS - 1) / ATTN_DECODE_MIN_KEYS;
     long ns = want;
     if (ns > by_len)
@@ -231,7 +239,7 @@ static void attn_run(const char *who, const uint16_t *Q, const uint16_t *K, cons
     if (attn_use_decode(Hkv, group, Sq)) {
         const int nrb = (group * Sq + ATTN_DECODE_ROWS - 1) / ATTN_DECODE_ROWS;
         int nsplit, kps;
-        attn_decode_split(Hq, Hkv, Sq, Sk, nrb, &nsplit, &kps);
+        attn_decode_split(Hq, Hkv, Sq, Sk, nrb, dp, &nsplit, &kps);
         struct attn_carve cv = {NULL, NULL, NULL};
         attn_layout(scratch, D, &cv);
         attn_hip_check(attn_hip_launch_decode(Q, K, V, O, cv.m, cv.l, cv.acc, Hq, Hkv, Sq, Sk, D,

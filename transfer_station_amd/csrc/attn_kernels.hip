@@ -21,10 +21,10 @@
 //                                          back (causal: pairs of a heavy and a light query
 //                                          tile), or (KH) one causal pair of 128-row items on
 //                                          key-tile halves
-//   attn_decode_kernel<DP,CAUSAL,VEC,VT>   split-K decode for g*Sq <= 64 rows per kv head
+//   attn_decode_kernel<DP,CAUSAL,VEC,VT,NTL,NRB> split-K decode for g*Sq <= 64 rows per kv head
 //   attn_decode_vt_kernel<DP,CAUSAL,NTL,UA> the same from V^T, staged in LDS 512 keys at a time
 //   attn_merge{2,w,}_kernel                log-sum-exp merge of split partials (2 splits / up to
-//                                          64, one wave per row / any, one workgroup per row)
+//                                          64 / any, one workgroup per row)
 //   attn_pack_v16_kernel<TK,VEC>           V [Hkv][Sk][D] -> V^T [Hkv][D][Sk]
 // VT selects a pre-transposed V ([Hkv][D][Sk], pack_v_full's layout).
 #include <hip/hip_runtime.h>
@@ -39,6 +39,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "attn_decode_rule.h"
 #include "attn_flash.h"
 
 namespace {
@@ -2092,6 +2093,68 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_persist_kernel(
 // dispatch); 4 floats of padding move each row 4 banks on, so the 16 lanes cover all 64.
 constexpr int kMergePad = 4;
 
+// The decode kernels' 4-wave merge of one 16-row block (its waves' o in om, their (m, l) in red_m and
+// red_l): rows row .. row + Mb - 1 of kv head u's g * Sq, into O (nsplit == 1) or the partial slots of
+// split sp. A thread takes 4 columns at a time: with single columns and a runtime division per
+// element, a 16-row block took 8 passes over 4 exponentials and two divisions each, which was
+// felt on short key ranges: 32 heads x 4 rows over 2000 keys at D = 64 9.2 -> 8.1 us, 128 kv heads x
+// 64 rows over 1000 keys 26.1 -> 23.9.
+template <int DP>
+__device__ __forceinline__ void decode_merge(const float *om, const float (*red_m)[16],
+                                             const float (*red_l)[16], float *__restrict__ O,
+                                             float *__restrict__ pm, float *__restrict__ pl,
+                                             float *__restrict__ pacc, int tid, int row, int Mb,
+                                             int u, int g, int Sq, int D, float c, int nsplit,
+                                             int sp) {
+    for (int idx = tid; idx < Mb * (DP / 4); idx += 256) {
+        const int r = idx / (DP / 4), d = 4 * (idx % (DP / 4));
+        if (d >= D)
+            continue;
+        float mx = kNegInf;
+#pragma unroll
+        for (int ww = 0; ww < 4; ++ww)
+            mx = fmaxf(mx, red_m[ww][r]);
+        const float muse = (mx == kNegInf) ? 0.f : mx;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        float lsum = 0.f;
+#pragma unroll
+        for (int ww = 0; ww < 4; ++ww) {
+            const float wgt = fast_exp2((red_m[ww][r] - muse) * c);
+            const f32x4 x =
+                *reinterpret_cast<const f32x4 *>(&om[(ww * 16 + r) * (DP + kMergePad) + d]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[j] += wgt * x[j];
+            lsum += wgt * red_l[ww][r];
+        }
+        const int gi = (row + r) / Sq;
+        const size_t orow = (size_t)(u * g + gi) * Sq + (row + r - gi * Sq);
+        float *dst;
+        if (nsplit == 1) {
+            const float inv = (lsum > 0.f) ? 1.0f / lsum : 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[j] *= inv;
+            dst = O + orow * D + d;
+        } else {
+            const size_t slot = orow * nsplit + sp;
+            if (d == 0) {
+                pm[slot] = mx;
+                pl[slot] = lsum;
+            }
+            dst = pacc + slot * D + d;
+        }
+        if (d + 4 <= D) {
+            *reinterpret_cast<f32x4_a4 *>(dst) = acc;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (d + j < D)
+                    dst[j] = acc[j];
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------------
 // Decode (split-K). One workgroup per (kv head u, split sp, 16-row block rb) serves up to 16 of
 // the M = g*Sq <= 64 query rows of that kv head from one read of its K/V range
@@ -2106,8 +2169,17 @@ constexpr int kMergePad = 4;
 // then loaded from global memory straight into its register layout, like K, with no LDS tile.
 // NTL: K and V are loaded non-temporally (decode_nt_loads decides).
 // ------------------------------------------------------------------------------------------
-template <int DP, bool CAUSAL, bool VEC, bool VT, bool NTL>
-__global__ __launch_bounds__(256) void attn_decode_kernel(
+// NRB: the row blocks one workgroup serves (rb counts groups of NRB); each K/V fragment is then read
+// once for all of them. Each row's arithmetic is that of NRB = 1. Two blocks for three or four of a
+// kv head (launch_decode_d): 64 rows over 4001 keys, 32 kv heads 28.6 -> 23.2 us, 128 kv heads over
+// 1000 keys 23.9 -> 21.9. Measured and not taken: four blocks at once (one wave per SIMD cannot cover
+// the load and MFMA latencies: 36.9 us), two blocks where there are two (24-32 heads' rows over 2000
+// keys at D = 64 8.1 -> 9.0 us: half the workgroups), the next step's loads issued a step ahead
+// (+5 to +12%, the registers take a wave per SIMD).
+// Two waves per SIMD are asked for; the 138 registers at D = 128 allow three (172 with no bound:
+// c2 162.4 -> 160 us, D = 256 with 8 kv heads 18.7 -> 14.9).
+template <int DP, bool CAUSAL, bool VEC, bool VT, bool NTL, int NRB>
+__global__ __launch_bounds__(256, 2) void attn_decode_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     const uint16_t *__restrict__ V, float *__restrict__ O, float *__restrict__ pm,
     float *__restrict__ pl, float *__restrict__ pacc, int Hq, int Hkv, int Sq, int Sk, int D,
@@ -2122,13 +2194,13 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
     constexpr int VNCH = 32 * DP / 8 / 64; // 16-byte chunks per lane per V tile
     constexpr int VTILE = 32 * VSTR;       // elements of one wave's V tile
     __shared__ __attribute__((aligned(16))) uint16_t Vw[4 * VTILE];
-    __shared__ float red_m[4][16], red_l[4][16];
+    __shared__ float red_m[NRB][4][16], red_l[NRB][4][16];
     // The 4-wave merge reuses the V tiles' memory as float [4][16][DP + 4] (kMergePad).
     static_assert(4 * 16 * (DP + kMergePad) * 4 <= 4 * VTILE * 2,
                   "merge area must fit in the V tiles");
 
-    // Block = (kv head u, split sp, row block rb): rows 16rb .. 16rb+15 of the kv head's M rows.
-    // Row blocks of one (u, sp) are consecutive logical ids, kept on one XCD so that they share
+    // Block = (kv head u, split sp, row block group rb): rows 16 NRB rb on of the kv head's M rows.
+    // Groups of one (u, sp) are consecutive logical ids, kept on one XCD so that they share
     // its L2 copy of the K/V range.
     const int g = Hq / Hkv, M = g * Sq;
     // The grid is Hkv * nsplit * nrb workgroups.
@@ -2138,27 +2210,32 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
     const int tid = wi_id_x(), w = tid >> 6, lane = tid & 63;
     const int r16 = lane & 15, grp = lane >> 4;
     const int k0 = sp * kps, k1 = min(k0 + kps, Sk);
-    const int row0 = 16 * rb, Mb = min(16, M - row0);
+    const int row0 = 16 * NRB * rb;
 
-    const bool rvalid = row0 + r16 < M;
-    const int gi = rvalid ? (row0 + r16) / Sq : 0, qi = rvalid ? (row0 + r16) % Sq : 0;
-    const int h = u * g + gi;
     const uint16_t *Kh = K + (size_t)u * Sk * D;
     const uint16_t *Vh = V + (size_t)u * Sk * D;
 
-    bf16x8 qb[DP / 32];
+    bf16x8 qb[NRB][DP / 32];
+    int lim[NRB];
+    float m_run[NRB], l_run[NRB];
+    f32x4 o[NRB][DP / 16];
 #pragma unroll
-    for (int kk = 0; kk < DP / 32; ++kk)
-        qb[kk] = as_bf16x8(
-            load_row8<VEC>(Q + (size_t)h * Sq * D, (size_t)qi, kk * 32 + grp * 8, D, rvalid,
-                           kk * 32 + 32));
-    const int lim = CAUSAL ? min(Sk - 1, Sk - Sq + qi) : Sk - 1;
-
-    float m_run = kNegInf, l_run = 0.f;
-    f32x4 o[DP / 16];
+    for (int b = 0; b < NRB; ++b) {
+        const int row = row0 + 16 * b + r16;
+        const bool rvalid = row < M;
+        const int gi = rvalid ? row / Sq : 0, qi = rvalid ? row % Sq : 0;
 #pragma unroll
-    for (int db = 0; db < DP / 16; ++db)
-        o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int kk = 0; kk < DP / 32; ++kk)
+            qb[b][kk] =
+                as_bf16x8(load_row8<VEC>(Q + (size_t)(u * g + gi) * Sq * D, (size_t)qi,
+                                         kk * 32 + grp * 8, D, rvalid, kk * 32 + 32));
+        lim[b] = CAUSAL ? min(Sk - 1, Sk - Sq + qi) : Sk - 1;
+        m_run[b] = kNegInf;
+        l_run[b] = 0.f;
+#pragma unroll
+        for (int db = 0; db < DP / 16; ++db)
+            o[b][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 
     uint16_t *vt = &Vw[w * VTILE];
     // Each workgroup starts its walk over the 128-key steps at a different step: workgroups
@@ -2166,142 +2243,147 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
     // 2*Sk-byte-strided rows over more HBM channels. attn_decode_vt_kernel walks the same order.
     const int nsteps = (k1 - k0 + 127) / 128;
     const int rot = us % (nsteps > 0 ? nsteps : 1);
-    for (int js = 0; js < nsteps; ++js) {
+    auto tile_of = [&](int js) {
         const int step = (js + rot < nsteps) ? js + rot : js + rot - nsteps;
-        const int tb = k0 + step * 128 + w * 32;
-        if (tb >= k1)
-            continue;
-        u32x4 ka[2][DP / 32];
+        return k0 + step * 128 + w * 32;
+    };
+    struct frags {
+        u32x4 k[2][DP / 32];
+        u32x4 v[VT ? DP / 16 : VNCH];
+    };
+    auto load = [&](int tb, frags &f) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const int key = tb + 8 * (r16 >> 2) + 4 * t + (r16 & 3);
 #pragma unroll
             for (int kk = 0; kk < DP / 32; ++kk)
-                ka[t][kk] = load_row8<VEC, NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1,
-                                                kk * 32 + 32);
+                f.k[t][kk] = load_row8<VEC, NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1,
+                                                 kk * 32 + 32);
         }
-        u32x4 vv[VT ? DP / 16 : VNCH];
         if (VT) {
             // lane: d row 16db + r16, keys tb + 8grp .. +7 (the k index of pk below).
 #pragma unroll
             for (int db = 0; db < DP / 16; ++db)
-                vv[db] = load_vt8<VEC, NTL>(Vh, db * 16 + r16, tb + 8 * grp, Sk, D, k1, tb + 32);
+                f.v[db] =
+                    load_vt8<VEC, NTL>(Vh, db * 16 + r16, tb + 8 * grp, Sk, D, k1, tb + 32);
         } else {
 #pragma unroll
             for (int r = 0; r < VNCH; ++r) {
                 const int cidx = lane + 64 * r;
                 const int row = cidx / (DP / 8), col = (cidx % (DP / 8)) * 8;
-                vv[r] = load_row8<VEC, NTL>(Vh, (size_t)(tb + row), col, D, tb + row < k1);
+                f.v[r] = load_row8<VEC, NTL>(Vh, (size_t)(tb + row), col, D, tb + row < k1);
             }
+        }
+    };
+    auto put_v = [&](const frags &f) __attribute__((always_inline)) {
+        if (!VT) {
             lds_wave_fence(); // previous tile's transposed reads are complete
 #pragma unroll
             for (int r = 0; r < VNCH; ++r) {
                 const int cidx = lane + 64 * r;
                 const int row = cidx / (DP / 8), col = (cidx % (DP / 8)) * 8;
                 const int colr = (col + VROT * ((row >> 3) & 1)) & (DP - 1);
-                *reinterpret_cast<u32x4 *>(&vt[row * VSTR + colr]) = vv[r];
+                *reinterpret_cast<u32x4 *>(&vt[row * VSTR + colr]) = f.v[r];
             }
         }
-        f32x4 s[2];
+    };
+    auto compute = [&](int tb, const frags &f) __attribute__((always_inline)) {
+        bf16x8 pk[NRB];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < NRB; ++b) {
+            f32x4 s[2];
 #pragma unroll
-            for (int kk = 0; kk < DP / 32; ++kk)
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[t][kk]), qb[kk], s[t], 0,
-                                                               0, 0);
-        }
-        // Register (t, i) of this lane holds key tb + 8grp + 4t + i for row r16.
-        float mx = kNegInf;
+            for (int t = 0; t < 2; ++t) {
+                s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = tb + 8 * grp + 4 * t + i;
-                if (key >= k1 || key > lim)
-                    s[t][i] = kNegInf;
-                mx = fmaxf(mx, s[t][i]);
+                for (int kk = 0; kk < DP / 32; ++kk)
+                    s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(f.k[t][kk]),
+                                                                   qb[b][kk], s[t], 0, 0, 0);
             }
-        mx = max_xor32(max_xor16(mx));
-        const float mnew = fmaxf(m_run, mx);
-        const float muse = (mnew == kNegInf) ? 0.f : mnew;
-        const float alpha = fast_exp2((m_run - muse) * c);
-        const float mc = muse * c;
-        float psum = 0.f;
-        bf16x8 pk;
+            // Register (t, i) of this lane holds key tb + 8grp + 4t + i for row r16.
+            float mx = kNegInf;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float p = fast_exp2(fmaf(s[t][i], c, -mc));
-                psum += p;
-                pk[4 * t + i] = (__bf16)p;
-            }
-        l_run = alpha * l_run + psum;
-        m_run = mnew;
+                for (int i = 0; i < 4; ++i) {
+                    const int key = tb + 8 * grp + 4 * t + i;
+                    if (key >= k1 || key > lim[b])
+                        s[t][i] = kNegInf;
+                    mx = fmaxf(mx, s[t][i]);
+                }
+            mx = max_xor32(max_xor16(mx));
+            const float mnew = fmaxf(m_run[b], mx);
+            const float muse = (mnew == kNegInf) ? 0.f : mnew;
+            const float alpha = fast_exp2((m_run[b] - muse) * c);
+            const float mc = muse * c;
+            float psum = 0.f;
 #pragma unroll
-        for (int db = 0; db < DP / 16; ++db)
-            o[db] *= alpha;
-        if (VT) {
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float p = fast_exp2(fmaf(s[t][i], c, -mc));
+                    psum += p;
+                    pk[b][4 * t + i] = (__bf16)p;
+                }
+            l_run[b] = alpha * l_run[b] + psum;
+            m_run[b] = mnew;
 #pragma unroll
             for (int db = 0; db < DP / 16; ++db)
-                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vv[db]), pk, o[db], 0, 0, 0);
-        } else {
+                o[b][db] *= alpha;
+        }
+        if (!VT)
             lds_wave_fence(); // this tile's V is in LDS before the transposed reads
-            // rows of this lane's reads: 8grp + r16/4 and 4 on, in row-octet grp
-            const int vrot = VROT * (grp & 1);
-            const uint16_t *vb0 = &vt[(8 * grp + (r16 >> 2)) * VSTR + 4 * (r16 & 3)];
+        // rows of this lane's reads: 8grp + r16/4 and 4 on, in row-octet grp
+        const int vrot = VROT * (grp & 1);
+        const uint16_t *vb0 = &vt[(8 * grp + (r16 >> 2)) * VSTR + 4 * (r16 & 3)];
 #pragma unroll
-            for (int db = 0; db < DP / 16; ++db) {
+        for (int db = 0; db < DP / 16; ++db) {
+            bf16x8 a;
+            if (VT) {
+                a = as_bf16x8(f.v[db < (int)(sizeof f.v / sizeof f.v[0]) ? db : 0]);
+            } else {
                 // column 16db + 4(r16 % 4) + vrot, modulo DP (db * 16 < DP - VROT: no wrap)
                 const uint16_t *vb = vb0 + db * 16 + ((db * 16 < DP - VROT) ? vrot : -vrot);
-                const bf16x8 a =
-                    join_tr(lds_read_tr(vb), lds_read_tr(vb + 4 * VSTR));
-                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pk, o[db], 0, 0, 0);
+                a = join_tr(lds_read_tr(vb), lds_read_tr(vb + 4 * VSTR));
             }
+#pragma unroll
+            for (int b = 0; b < NRB; ++b)
+                o[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pk[b], o[b][db], 0, 0, 0);
         }
+    };
+    for (int js = 0; js < nsteps; ++js) {
+        const int tb = tile_of(js);
+        if (tb >= k1)
+            continue;
+        frags f;
+        load(tb, f);
+        put_v(f);
+        compute(tb, f);
     }
-    l_run = sum_xor32(sum_xor16(l_run));
+#pragma unroll
+    for (int b = 0; b < NRB; ++b)
+        l_run[b] = sum_xor32(sum_xor16(l_run[b]));
 
     // Merge the 4 waves: O^T register (db, i) of this lane holds d = 16db + 4grp + i, row r16.
-    __syncthreads();
     float *om = reinterpret_cast<float *>(Vw); // [4][16][DP + kMergePad]
-    if (grp == 0) {
-        red_m[w][r16] = m_run;
-        red_l[w][r16] = l_run;
-    }
+    if (grp == 0)
 #pragma unroll
-    for (int db = 0; db < DP / 16; ++db)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            om[(w * 16 + r16) * (DP + kMergePad) + db * 16 + 4 * grp + i] = o[db][i];
-    __syncthreads();
-    for (int idx = tid; idx < Mb * D; idx += 256) {
-        const int r = idx / D, d = idx - r * D;
-        float mx = kNegInf;
-#pragma unroll
-        for (int ww = 0; ww < 4; ++ww)
-            mx = fmaxf(mx, red_m[ww][r]);
-        const float muse = (mx == kNegInf) ? 0.f : mx;
-        float acc = 0.f, lsum = 0.f;
-#pragma unroll
-        for (int ww = 0; ww < 4; ++ww) {
-            const float wgt = fast_exp2((red_m[ww][r] - muse) * c);
-            acc += wgt * om[(ww * 16 + r) * (DP + kMergePad) + d];
-            lsum += wgt * red_l[ww][r];
+        for (int b = 0; b < NRB; ++b) {
+            red_m[b][w][r16] = m_run[b];
+            red_l[b][w][r16] = l_run[b];
         }
-        const int hr = u * g + (row0 + r) / Sq, qr = (row0 + r) % Sq;
-        const size_t orow = (size_t)hr * Sq + qr;
-        if (nsplit == 1) {
-            O[orow * D + d] = acc * ((lsum > 0.f) ? 1.0f / lsum : 0.f);
-        } else {
-            const size_t slot = orow * nsplit + sp;
-            pacc[slot * D + d] = acc;
-            if (d == 0) {
-                pm[slot] = mx;
-                pl[slot] = lsum;
-            }
-        }
+#pragma unroll
+    for (int b = 0; b < NRB; ++b) {
+        __syncthreads();
+#pragma unroll
+        for (int db = 0; db < DP / 16; ++db)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                om[(w * 16 + r16) * (DP + kMergePad) + db * 16 + 4 * grp + i] = o[b][db][i];
+        __syncthreads();
+        const int rowb = row0 + 16 * b, Mb = min(16, M - rowb);
+        decode_merge<DP>(om, red_m[b], red_l[b], O, pm, pl, pacc, tid, rowb, Mb, u, g, Sq, D, c,
+                         nsplit, sp);
     }
 }
 
@@ -2556,33 +2638,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
         for (int i = 0; i < 4; ++i)
             om[(w * 16 + r16) * (DP + kMergePad) + db * 16 + 4 * grp + i] = o[db][i];
     __syncthreads();
-    for (int idx = tid; idx < Mb * D; idx += 256) {
-        const int r = idx / D, d = idx - r * D;
-        float mx = kNegInf;
-#pragma unroll
-        for (int ww = 0; ww < 4; ++ww)
-            mx = fmaxf(mx, red_m[ww][r]);
-        const float muse = (mx == kNegInf) ? 0.f : mx;
-        float acc = 0.f, lsum = 0.f;
-#pragma unroll
-        for (int ww = 0; ww < 4; ++ww) {
-            const float wgt = fast_exp2((red_m[ww][r] - muse) * c);
-            acc += wgt * om[(ww * 16 + r) * (DP + kMergePad) + d];
-            lsum += wgt * red_l[ww][r];
-        }
-        const int hr = u * g + (row0 + r) / Sq, qr = (row0 + r) % Sq;
-        const size_t orow = (size_t)hr * Sq + qr;
-        if (nsplit == 1) {
-            O[orow * D + d] = acc * ((lsum > 0.f) ? 1.0f / lsum : 0.f);
-        } else {
-            const size_t slot = orow * nsplit + sp;
-            pacc[slot * D + d] = acc;
-            if (d == 0) {
-                pm[slot] = mx;
-                pl[slot] = lsum;
-            }
-        }
-    }
+    decode_merge<DP>(om, red_m, red_l, O, pm, pl, pacc, tid, row0, Mb, u, g, Sq, D, c, nsplit, sp);
 }
 
 // Merge of split-K partials. Partial row r owns slots r*nsplit .. r*nsplit+nsplit-1 and covers
@@ -2662,59 +2718,111 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
     }
 }
 
-// 3 <= nsplit <= kMergeWaveMaxSplit (the prefill key split and short decode splits): one wave per
-// partial row, 4 rows per workgroup. Lane s holds split s's (m, l); the max and the weighted l
-// sum are wave reductions, and the final weights w_s / sum go through LDS to every lane. Columns
-// are float2 where D is even and O 8-byte aligned, so each split's columns are one coalesced
-// read per wave. Waves past the last row still reach the barrier.
+// 3 <= nsplit <= kMergeWaveMaxSplit (the prefill key split and decode splits): lp lanes cover a
+// row's columns in 4-float pieces (lp a power of two, 4 lp >= D) and ng groups of them its splits,
+// so a row takes lp * ng threads and a workgroup 256 / (lp ng) rows. Each thread issues its splits'
+// loads (kMergeLoads at a time) before the weights are known; the weights (one wave per row: max and
+// weighted l sum over its lanes) go through LDS, the groups' sums too. With few rows and many
+// splits the launch is latency-bound: one wave per row reading its splits one by one took 7.2 us
+// for 32 rows x 64 splits at D = 128 (8 workgroups); decode over 32768 keys 30.6 -> 26.9 us with this
+// layout, over 777 keys 9.5 -> 8.8.
 constexpr int kMergeWaveMaxSplit = 64;
+constexpr int kMergeLoads = 8;
+// max or sum over the wave's 64 lanes, in every lane, on the VALU.
+template <bool MAX> __device__ __forceinline__ float wave_all(float x) {
+    auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+    auto ror = [](float v, auto C) {
+        const int u = __builtin_bit_cast(int, v);
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_update_dpp(u, u, decltype(C)::value, 0xf, 0xf, false));
+    };
+    x = op(x, ror(x, std::integral_constant<int, 0x128>{})); // row_ror:8, 4, 2, 1
+    x = op(x, ror(x, std::integral_constant<int, 0x124>{}));
+    x = op(x, ror(x, std::integral_constant<int, 0x122>{}));
+    x = op(x, ror(x, std::integral_constant<int, 0x121>{}));
+    return MAX ? max_xor32(max_xor16(x)) : sum_xor32(sum_xor16(x));
+}
 __global__ __launch_bounds__(256) void attn_mergew_kernel(const float *__restrict__ pm,
                                                           const float *__restrict__ pl,
                                                           const float *__restrict__ pacc,
                                                           float *__restrict__ O, long rows, int D,
                                                           int nsplit, float c, int rph, int q_off,
-                                                          int Sq) {
-    typedef __attribute__((ext_vector_type(2))) float f32x2;
-    __shared__ float wsh[4][kMergeWaveMaxSplit];
-    const int wv = wi_id_x() >> 6, lane = wi_id_x() & 63;
-    const long row = (long)wg_id_x() * 4 + wv;
-    const bool valid = row < rows;
-    const bool mine = valid && lane < nsplit;
-    const float ms = mine ? pm[row * nsplit + lane] : kNegInf;
-    float mx = ms;
+                                                          int Sq, int lp, int ng) {
+    __shared__ float wsh[32][kMergeWaveMaxSplit]; // up to 32 rows (lp = 8: D <= 32)
+    __shared__ __attribute__((aligned(16))) f32x4 red[256];
+    const int tid = wi_id_x(), wv = tid >> 6, lane = tid & 63;
+    const int tpr = lp * ng, rpw = 256 / tpr;
+    const long row0 = (long)wg_id_x() * rpw;
+    const int rl = tid / tpr, t = tid - rl * tpr; // the thread's row of the workgroup, lane in it
+    const int g = t / lp, d = 4 * (t - g * lp);
+    const long row = row0 + rl;
+    const bool mine = row < rows && d < D;
+    const float *pr = pacc + (size_t)row * nsplit * D + d;
+    auto piece = [&](int s) -> f32x4 {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (mine && s < nsplit) {
+            const float *p = pr + (size_t)s * D;
+            if (d + 4 <= D) {
+                v = *reinterpret_cast<const f32x4_a4 *>(p);
+            } else {
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1)
-        mx = fmaxf(mx, __shfl_xor(mx, o));
-    const float muse = (mx == kNegInf) ? 0.f : mx;
-    const float w = mine ? fast_exp2((ms - muse) * c) : 0.f;
-    float lw = mine ? w * pl[row * nsplit + lane] : 0.f;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1)
-        lw += __shfl_xor(lw, o);
-    wsh[wv][lane] = w * ((lw > 0.f) ? 1.0f / lw : 0.f);
-    __syncthreads();
-    if (!valid)
-        return;
-    const float *pr = pacc + (size_t)row * nsplit * D;
-    float *o = O + merge_orow(row, rph, q_off, Sq) * D;
-    if ((D & 1) == 0 && ((uintptr_t)O & 7u) == 0) {
-        for (int d = 2 * lane; d < D; d += 128) {
-            f32x2 acc = {0.f, 0.f};
-            for (int sp = 0; sp < nsplit; ++sp) {
-                const float a = wsh[wv][sp];
-                const f32x2 x = *reinterpret_cast<const f32x2 *>(pr + (size_t)sp * D + d);
-                acc[0] += a * x[0];
-                acc[1] += a * x[1];
+                for (int j = 0; j < 3; ++j)
+                    if (d + j < D)
+                        v[j] = p[j];
             }
-            *reinterpret_cast<f32x2 *>(o + d) = acc;
         }
+        return v;
+    };
+    f32x4 x[kMergeLoads];
+#pragma unroll
+    for (int i = 0; i < kMergeLoads; ++i)
+        x[i] = piece(g + i * ng);
+    for (int r = wv; r < rpw; r += 4) {
+        const bool in = row0 + r < rows && lane < nsplit;
+        const size_t slot = (size_t)(row0 + r) * nsplit + lane;
+        const float ms = in ? pm[slot] : kNegInf;
+        const float ls = in ? pl[slot] : 0.f;
+        const float mx = wave_all<true>(ms);
+        const float muse = (mx == kNegInf) ? 0.f : mx;
+        const float w = in ? fast_exp2((ms - muse) * c) : 0.f;
+        const float lw = wave_all<false>(w * ls);
+        wsh[r][lane] = w * ((lw > 0.f) ? 1.0f / lw : 0.f);
+    }
+    __syncthreads();
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < nsplit; s0 += kMergeLoads * ng) {
+#pragma unroll
+        for (int i = 0; i < kMergeLoads; ++i) {
+            const int s = s0 + g + i * ng;
+            const float a = s < nsplit ? wsh[rl][s] : 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[j] += a * x[i][j];
+            x[i] = piece(s + kMergeLoads * ng);
+        }
+    }
+    if (ng > 1) {
+        red[tid] = acc;
+        __syncthreads();
+        if (g != 0)
+            return;
+        for (int k = 1; k < ng; ++k) {
+            const f32x4 y = red[tid + k * lp];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[j] += y[j];
+        }
+    }
+    if (!mine)
+        return;
+    float *o = O + merge_orow(row, rph, q_off, Sq) * D + d;
+    if (d + 4 <= D) {
+        *reinterpret_cast<f32x4_a4 *>(o) = acc;
     } else {
-        for (int d = lane; d < D; d += 64) {
-            float acc = 0.f;
-            for (int sp = 0; sp < nsplit; ++sp)
-                acc += wsh[wv][sp] * pr[(size_t)sp * D + d];
-            o[d] = acc;
-        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (d + j < D)
+                o[j] = acc[j];
     }
 }
 
@@ -2865,6 +2973,22 @@ __attribute__((format(printf, 3, 4))) void plan_note(dim3 g, dim3 b, const char 
     p->buf[p->pos] = '\0';
 }
 
+// Compute units of the current device (cached per device).
+static int device_cus() {
+    static int cus[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
+        return 256;
+    if (cus[dev] <= 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            n <= 0)
+            n = 256;
+        cus[dev] = n;
+    }
+    return cus[dev];
+}
+
 hipError_t launch_merge(const float *pm, const float *pl, const float *pacc, float *O, long rows,
                         int D, int nsplit, float c, int rph, int q_off, int Sq, hipStream_t st) {
     if (rows <= 0 || rows > 0x7fffffffL || rph <= 0)
@@ -2881,13 +3005,22 @@ hipError_t launch_merge(const float *pm, const float *pl, const float *pacc, flo
             hipLaunchKernelGGL(attn_merge2_kernel, dim3((unsigned)((rows + rpw - 1) / rpw)),
                                dim3(256), 0, st, pm, pl, pacc, O, rows, D, c, rph, q_off, Sq, lpr);
     }
-    else if (nsplit <= kMergeWaveMaxSplit) {
+    else if (nsplit <= kMergeWaveMaxSplit && D <= 256) {
+        int lp = 8;
+        while (4 * lp < D)
+            lp *= 2;
+        // Split groups per row: at most kMergeLoads loads per thread where the workgroup allows, and
+        // more groups (down to two loads per thread) while the grid has fewer threads than the GPU.
+        int ng = 1;
+        while (2 * ng * lp <= 256 && (ng * kMergeLoads < nsplit ||
+                                      (4 * ng <= nsplit && rows * lp * ng < 256L * device_cus())))
+            ng *= 2;
+        const long nwg = (rows + 256 / (lp * ng) - 1) / (256 / (lp * ng));
         if (t_plan)
-            plan_note(dim3((unsigned)((rows + 3) / 4)), dim3(256), "attn_mergew_kernel nsplit=%d",
-                      nsplit);
+            plan_note(dim3((unsigned)nwg), dim3(256), "attn_mergew_kernel nsplit=%d", nsplit);
         else
-            hipLaunchKernelGGL(attn_mergew_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
-                               st, pm, pl, pacc, O, rows, D, nsplit, c, rph, q_off, Sq);
+            hipLaunchKernelGGL(attn_mergew_kernel, dim3((unsigned)nwg), dim3(256), 0, st, pm, pl,
+                               pacc, O, rows, D, nsplit, c, rph, q_off, Sq, lp, ng);
     } else if (nsplit <= kMergeMaxSplit && D <= 256) {
         if (t_plan)
             plan_note(dim3((unsigned)rows), dim3(256), "attn_merge_kernel nsplit=%d", nsplit);
@@ -2898,22 +3031,6 @@ hipError_t launch_merge(const float *pm, const float *pl, const float *pacc, flo
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
-}
-
-// Compute units of the current device (cached per device).
-static int device_cus() {
-    static int cus[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
-        return 256;
-    if (cus[dev] <= 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            n <= 0)
-            n = 256;
-        cus[dev] = n;
-    }
-    return cus[dev];
 }
 
 // Short query blocks under GQA (Sq <= 64, g > 1): the g heads' rows of a kv head share query
@@ -3425,9 +3542,16 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
     if (nblk <= 0 || nblk > 0x7fffffffL)
         return hipErrorInvalidValue;
     const bool ntl = decode_nt_loads(nrb, kps);
-    // The staged V^T kernel's DMA offsets are 32-bit: a head's V^T must stay below 2 GiB.
+    const int blocks = attn_decode_blocks(nrb, DP, Hkv, Sk);
+    // The staged V^T kernel, for one row block per workgroup and more than one 128-key step: its
+    // pipeline fills over five barrier intervals (8 kv heads over 776 keys in one-step splits 10.3 us,
+    // attn_decode_kernel straight from V^T 8.2; over 777 keys 14.2 and 10.0; two steps and up it is
+    // the faster one, 64 kv heads over 3001 keys 24.0 and 28.0). Its DMA offsets are 32-bit: a head's
+    // aligned V^T must stay below 2 GiB. Grouped row blocks read V^T once straight from memory (32 kv
+    // heads, 64 rows over 4000 keys: staged per block 33, this 25.5).
     if constexpr (DP <= 128)
-        if (vt && decode_vt_staged() && (vec ? (long)D * Sk * 2 < 0x7fffffffL : Sk >= 8))
+        if (vt && blocks == 1 && kps > ATTN_DECODE_MIN_KEYS && decode_vt_staged() &&
+            (vec ? (long)D * Sk * 2 < 0x7fffffffL : Sk >= 8))
             return with_flag(causal != 0, [&](auto CA) {
                 return with_flag(ntl, [&](auto NT) {
                     return with_flag(vec == 0, [&](auto UAF) {
@@ -3446,26 +3570,36 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
                     });
                 });
             });
-    return with_flag(causal != 0, [&](auto CA) {
-        return with_flag(vec != 0, [&](auto VE) {
-            return with_flag(vt != 0, [&](auto VTF) {
-                return with_flag(ntl, [&](auto NT) {
-                    if (t_plan)
-                        plan_note(dim3((unsigned)nblk), dim3(256),
-                                  "attn_decode_kernel<%d, %s, %s, %s, %s> nsplit=%d nrb=%d", DP,
-                                  tf(decltype(CA)::value), tf(decltype(VE)::value),
-                                  tf(decltype(VTF)::value), tf(decltype(NT)::value), nsplit, nrb);
-                    else
-                        hipLaunchKernelGGL(
-                            (attn_decode_kernel<DP, decltype(CA)::value, decltype(VE)::value,
-                                                decltype(VTF)::value, decltype(NT)::value>),
-                            dim3((unsigned)nblk), dim3(256), 0, st, Q, K, V, O, pm, pl, pacc, Hq,
-                            Hkv, Sq, Sk, D, c, nsplit, kps, nrb);
-                    return hipGetLastError();
+    auto go = [&](auto NB) {
+        constexpr int NRB = decltype(NB)::value;
+        const int ng = (nrb + NRB - 1) / NRB; // row block groups
+        const long n = (long)Hkv * nsplit * ng;
+        return with_flag(causal != 0, [&](auto CA) {
+            return with_flag(vec != 0, [&](auto VE) {
+                return with_flag(vt != 0, [&](auto VTF) {
+                    return with_flag(ntl, [&](auto NT) {
+                        constexpr bool kC = decltype(CA)::value, kE = decltype(VE)::value,
+                                       kT = decltype(VTF)::value, kN = decltype(NT)::value;
+                        if (t_plan)
+                            plan_note(dim3((unsigned)n), dim3(256),
+                                      "attn_decode_kernel<%d, %s, %s, %s, %s%s> nsplit=%d nrb=%d",
+                                      DP, tf(kC), tf(kE), tf(kT), tf(kN),
+                                      NRB == 2 ? ", 2 blocks" : "",
+                                      nsplit, nrb);
+                        else
+                            hipLaunchKernelGGL((attn_decode_kernel<DP, kC, kE, kT, kN, NRB>),
+                                               dim3((unsigned)n), dim3(256), 0, st, Q, K, V, O, pm,
+                                               pl, pacc, Hq, Hkv, Sq, Sk, D, c, nsplit, kps, ng);
+                        return hipGetLastError();
+                    });
                 });
             });
         });
-    });
+    };
+    if constexpr (DP <= 128)
+        if (blocks == 2)
+            return go(std::integral_constant<int, 2>{});
+    return go(std::integral_constant<int, 1>{});
 }
 
 } // namespace
