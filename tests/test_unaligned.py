@@ -104,6 +104,13 @@ def test_unaligned_pack(Hkv, Sk, D):
     # Hq, Hkv, Sq, Sk, D, causal: 192-wide tiles (D in (128, 192]) and the last of the 256-wide
     (8, 2, 300, 640, 136, 0), (8, 2, 300, 640, 192, 1), (8, 2, 300, 640, 200, 1),
     (6, 3, 129, 65, 160, 0), (16, 4, 40, 129, 184, 1),
+    # 8 waves: tiles of 32 keys (D > 192) and 64, whole and ragged, one to many of them
+    (48, 8, 700, 200, 256, 0), (160, 16, 700, 700, 200, 1), (72, 8, 400, 832, 256, 1),
+    (48, 8, 700, 24, 256, 0), (256, 32, 256, 40, 208, 0), (48, 8, 700, 328, 136, 0),
+    (160, 16, 641, 648, 192, 1), (256, 32, 256, 64, 192, 0),
+    # and without the vector layout
+    (4, 2, 257, 333, 189, 0), (4, 2, 300, 301, 250, 1), (2, 1, 129, 5, 201, 0), (3, 1, 500, 77, 131, 1),
+    (256, 16, 500, 507, 256, 1),
 ])
 def test_wide_head_dims(oracle, case):
     """The wide tiles' loop without a rescale, and its way out: keys whose scores jump from tile to
@@ -118,6 +125,10 @@ def test_wide_head_dims(oracle, case):
     R = oracle.attn_ref(Q, K.ravel(), V, Hq, Hkv, Sq, Sk, D, causal, rows, nthreads=8)
     for vt in (0, 1):
         Vin = np.ascontiguousarray(V.reshape(Hkv, Sk, D).transpose(0, 2, 1)).ravel() if vt else V
+        if Hq >= 48 or D % 8:  # the 8-wave cases
+            kt = 64 if D <= 192 and D % 8 == 0 and not (vt and Sk % 8) else 32
+            name = ts.attn_flash_plan(Hq, Hkv, Sq, Sk, D, causal, v_prepacked=vt)[0][0]
+            assert "<%d, %d, 8, " % (192 if D <= 192 else 256, kt) in name, (case, vt, name)
         O = attend(Q, K.ravel(), Vin, Hq, Hkv, Sq, Sk, D, causal, vt, 0)
         ok, mad, maxref, nbad = oracle.cmp_rows(R, O, Hq, Sq, D, rows)
         print("   vt=%d err/scale=%.2e nbad=%d" % (vt, mad / maxref, nbad), flush=True)

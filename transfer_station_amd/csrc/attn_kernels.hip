@@ -377,7 +377,7 @@ constexpr int prefill_wg_per_cu(int DP, int KT, int NW) {
 // start of the tile before, put into LDS at its end. What bounds it is those loads (2-byte aligned
 // ones cost 6% more than 4-byte aligned ones, which cost what 16-byte aligned ones do), the registers
 // they hold (two pieces per thread and tensor on 64-key tiles at 8 waves; on 4 waves, or K waited
-// for in mid-tile, 27-75% slower) and the row max, which every tile takes: the largest weights
+// for in mid-tile, 27-75% slower; D > 128 on 8 waves: kRing below) and the row max, which every tile takes: the largest weights
 // of a row are then exactly 1 or close below (error against 64 bits 1.5e-3 of the result, 1.7e-3
 // with the sum test, which was 8% faster). Same box, element-wise loads before -> now: 24 heads of
 // 1000 rows over 2003 keys, D = 100, V^T with its pack 249 -> 57 us; 64 heads at 2k, D = 128, V^T
@@ -396,6 +396,16 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
                   "key halves: 8 waves (or 12 at DP = 64), 128-key tiles");
     static_assert(NW != 12 || KH, "12 waves: key halves only");
     // Software-pipelined tiles (tile_pipelined): D <= 64, key halves on 12 waves only.
+    // 8 waves at DP > 128: two waves per SIMD of 256 registers each, 128 (96) of them O and 64 (48)
+    // Q, where 4 waves have 512. What made room: K and V fragments go through a ring of RD, read RD
+    // MFMAs ahead, instead of a whole sub-tile's and chunk's, and at DP = 256 (and unaligned) a tile is
+    // 32 keys; RD is what fits (aligned: no spills; unaligned at 256: 5). One wave's softmax and LDS
+    // latency then runs under the other's MFMAs, and a tile is read from L2 for 256 rows. Same
+    // box, 4 -> 8 waves, 64 heads at 2k: D = 256 282 -> 232 us (1185 TFLOP/s), causal 160 -> 136, V^T
+    // 322 -> 238, D = 192 220 -> 184; unaligned, D = 189 over 2003 keys 530 -> 253, D = 250 at 1000
+    // rows 307 -> 154. Bound as the 8-wave kernels at DP = 128 are: LDS reads beside the MFMAs.
+    constexpr bool kRing = DP > 128 && NW == 8;
+    constexpr int RD = !kRing ? 1 : DP < 256 ? 4 : UA ? 2 : VT ? 3 : 4;
     constexpr bool kPipe = DP <= 64 && (!KH || NW == 12) && !UA;
     constexpr int NR = KH ? NW / 2 : NW; // waves with distinct query rows
     constexpr int KW = KH ? KT / 2 : KT; // keys of a tile that one wave takes
@@ -782,6 +792,36 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     // fragments are read between this sub-tile's MFMAs.
     auto qk = [&](int buf) __attribute__((always_inline)) {
         const uint16_t *kb0 = &Ks[buf][kfo + kh * (KW / 32) * KSUB];
+        if constexpr (kRing) {
+            constexpr int NK = DP / 16, N = KW / 32 * NK;
+            auto frag = [&](int f) {
+                return as_bf16x8(
+                    *reinterpret_cast<const u32x4 *>(kb0 + f / NK * KSUB + f % NK * KDK));
+            };
+            bf16x8 kr[RD];
+#pragma unroll
+            for (int f = 0; f < RD; ++f)
+                kr[f] = frag(f);
+            __builtin_amdgcn_sched_group_barrier(0x100, RD, 0);
+#pragma unroll
+            for (int f = 0; f < N; ++f) {
+                if (f % NK == 0)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        s[f / NK][i] = 0.f;
+                s[f / NK] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kr[f % RD], qb[f % NK],
+                                                                   s[f / NK], 0, 0, 0);
+                if (f + RD < N)
+                    kr[f % RD] = frag(f + RD);
+            }
+#pragma unroll
+            for (int f = 0; f < N; ++f) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (f + RD < N)
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+            return;
+        }
         bf16x8 ka[2][DP / 16];
 #pragma unroll
         for (int kk = 0; kk < DP / 16; ++kk)
@@ -901,7 +941,14 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         const uint16_t *vb = &Vs[buf][vfo + cc * 16 * DP + db * 128];
         return join_tr(lds_read_tr(vb), lds_read_tr(vb + 4 * DP));
     };
+    bf16x8 vr[RD];
     auto pv_first = [&](int buf) {
+        if constexpr (kRing) {
+#pragma unroll
+            for (int f = 0; f < RD; ++f)
+                vr[f] = vfrag(buf, f / (DP / 32), f % (DP / 32));
+            return;
+        }
 #pragma unroll
         for (int db = 0; db < DP / 32; ++db)
             va[0][db] = vfrag(buf, 0, db);
@@ -928,6 +975,23 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         l_run += psum;
     };
     auto pv = [&](int buf) {
+        if constexpr (kRing) {
+            constexpr int ND = DP / 32, N = KW / 16 * ND;
+#pragma unroll
+            for (int f = 0; f < N; ++f) {
+                o[f % ND] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vr[f % RD], pk[f / ND],
+                                                                   o[f % ND], 0, 0, 0);
+                if (f + RD < N)
+                    vr[f % RD] = vfrag(buf, (f + RD) / ND, (f + RD) % ND);
+            }
+#pragma unroll
+            for (int f = 0; f < N; ++f) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (f + RD < N)
+                    __builtin_amdgcn_sched_group_barrier(0x100, VT ? 1 : 2, 0);
+            }
+            return;
+        }
 #pragma unroll
         for (int cc = 0; cc < KW / 16; ++cc) {
 #pragma unroll
@@ -1146,8 +1210,15 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
             __syncthreads();
         }
     };
+    // kRing on 32-key tiles: the first two take the row max, so that m starts at the largest of 64
+    // keys as on 64-key tiles (with one, causal errors against 64 bits grew from 1.33e-3 to 1.36e-3;
+    // with two they are 1.32e-3).
+    constexpr int NF = kRing && KT == 32 && !UA ? 2 : 1;
     if (kt0 < kt1)
         step(kt0, std::true_type{}, std::true_type{});
+    if constexpr (NF == 2)
+        if (kt0 + 1 < kt1)
+            step(kt0 + 1, std::true_type{}, std::true_type{});
     phase_stamp(w, lane, 2);
     if constexpr (DP > 128 && !UA) {
         // Unmasked tiles in a loop with no rescale of O in it: with 512 registers O lives in
@@ -1155,8 +1226,8 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         // all of O out of them on every tile (128 v_accvgpr_read per 64-key tile at DP = 256). A
         // tile whose sum test fails leaves the loop, takes the row max outside and comes back.
         // Bit-identical; same box, 64 heads at 2k: D = 256 323 -> 295 us (933 TFLOP/s), causal
-        // 194 -> 179. One wave per SIMD bounds it: its softmax, LDS reads and MFMAs take turns
-        // (MFMA busy 35% of the clocks). Software-pipelined sub-tiles (8 or 12 fragments ahead)
+        // 194 -> 179. At 4 waves one wave per SIMD bounds it: its softmax, LDS reads and MFMAs take
+        // turns (MFMA busy 35% of the clocks). Software-pipelined sub-tiles (8 or 12 fragments ahead)
         // measured 10% slower than these plain phases, alternating the two Q.K^T accumulators
         // within 1%.
         const int medge = CAUSAL ? min(Sk - KT, Sk - Sq + qmin - KT + 1) : Sk - KT;
@@ -1169,7 +1240,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
                 __syncthreads();
             }
         };
-        int kt = kt0 + 1;
+        int kt = kt0 + NF;
         for (;;) {
             bool redo = false;
             for (; kt < kt_m; ++kt) {
@@ -3374,6 +3445,35 @@ hipError_t launch_prefill_persist(const uint16_t *Q, const uint16_t *K, const ui
     return hipGetLastError();
 }
 
+// 8 waves at D > 128 (attn_prefill_fast_kernel's kRing) instead of 4; either way a CU holds one
+// workgroup. A round of 256-row workgroups takes 1.67 times a round of 128-row ones (D = 256 and 192,
+// 64 heads at 2k), so 8 waves are taken where their rounds are under 4/7 of the others': 36 heads of 1024
+// rows, D = 192, 103 -> 72 us, 128 heads of 400 rows 50 -> 38; one round either way (32
+// heads of 1000 rows, D = 256) 77 with 4 waves, 85 with 8. Not where 256-row tiles are padded much more
+// (300 rows, 128 heads: 213 and 218). Triangular causal grids are balanced heaviest first, down to
+// their longest item: 8 waves where the larger of that and the mean load falls under 3/4 (48 heads
+// at 2k 122 -> 106 us; 24 heads 70 with 4 waves, 88 with 8; 16 heads at 4k 141 and 159).
+// Unaligned tensors (ua): a round takes the same time with both, so 8 waves wherever they
+// need fewer tiles (16 heads of 200 rows 27.6 -> 28.6 us, 24 heads of 300 47 -> 43, of 1500 causal
+// 100 -> 68, 4 heads of 700 over 5000 keys 68 -> 54).
+static bool prefill_wide8(int Hq, int Hkv, int Sq, int Sk, bool causal, bool ua = false) {
+    if (const int forced = prefill_waves_forced())
+        return forced == 8;
+    if (prefill_pack(Hq, Hkv, Sq))
+        return false;
+    const long cus = device_cus();
+    const long t4 = (Sq + 127) / 128, t8 = (Sq + 255) / 256, n4 = Hq * t4, n8 = Hq * t8;
+    if (ua)
+        return t8 < t4;
+    if (8 * t8 > 5 * t4)
+        return false;
+    if (causal && (long)Sk - Sq < Sq) {
+        auto load = [&](long n) { return max((long)Sk * cus, n * (Sk - Sq / 2)); };
+        return 4 * load(n8) < 3 * load(n4);
+    }
+    return 7 * ((n8 + cus - 1) / cus) < 4 * ((n4 + cus - 1) / cus);
+}
+
 template <int DP, int KT, bool CAUSAL, bool VT>
 hipError_t launch_prefill_fast_t(const uint16_t *Q, const uint16_t *K, const uint16_t *V, float *O,
                                  int Hq, int Hkv, int Sq, int Sk, int D, float c, float *pm,
@@ -3431,9 +3531,13 @@ hipError_t launch_prefill_fast_t(const uint16_t *Q, const uint16_t *K, const uin
         if (nw == 8)
             return launch_prefill_fast_nw<DP, KT, 8, CAUSAL, VT>(Q, K, V, O, Hq, Hkv, Sq, Sk, D, c,
                                                                  pm, pl, pacc, slots, st);
+    if constexpr (DP > 128)
+        if (prefill_wide8(Hq, Hkv, Sq, Sk, CAUSAL))
+            return launch_prefill_fast_nw<DP, DP == 192 ? 64 : 32, 8, CAUSAL, VT>(
+                Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm, pl, pacc, slots, st);
     // 4-wave workgroups at D > 64 take 64-key tiles: at 128 keys the tiles use 96-128 KB of LDS
-    // and a CU could hold only one such workgroup (one wave per SIMD). At D > 128 the O and Q
-    // registers allow only one wave per SIMD anyway, so that is the only shape there.
+    // and a CU could hold only one such workgroup (one wave per SIMD). At D > 128 the grids that
+    // prefill_wide8 leaves take them, one workgroup per CU.
     return launch_prefill_fast_nw<DP, KT4, 4, CAUSAL, VT>(Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm,
                                                           pl, pacc, slots, st);
 }
@@ -3458,6 +3562,10 @@ hipError_t launch_prefill_ua(const uint16_t *Q, const uint16_t *K, const uint16_
             return launch_prefill_fast_nw<DP, KT4, 8, CAUSAL, VT, false, 1>(
                 Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm, pl, pacc, slots, st);
     }
+    if constexpr (DP > 128)
+        if (prefill_wide8(Hq, Hkv, Sq, Sk, CAUSAL, true))
+            return launch_prefill_fast_nw<DP, KT4, 8, CAUSAL, VT, false, 1>(
+                Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm, pl, pacc, slots, st);
     return launch_prefill_fast_nw<DP, KT4, 4, CAUSAL, VT, false, 1>(
         Q, K, V, O, Hq, Hkv, Sq, Sk, D, c, pm, pl, pacc, slots, st);
 }
