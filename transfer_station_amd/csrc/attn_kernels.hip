@@ -3468,7 +3468,8 @@ static bool prefill_wide8(int Hq, int Hkv, int Sq, int Sk, bool causal, bool ua 
     if (8 * t8 > 5 * t4)
         return false;
     if (causal && (long)Sk - Sq < Sq) {
-        auto load = [&](long n) { return max((long)Sk * cus, n * (Sk - Sq / 2)); };
+        // std::max: HIP's host max takes int, and these products pass 2^31.
+        auto load = [&](long n) { return std::max((long)Sk * cus, n * (Sk - Sq / 2)); };
         return 4 * load(n8) < 3 * load(n4);
     }
     return 7 * ((n8 + cus - 1) / cus) < 4 * ((n4 + cus - 1) / cus);
@@ -3819,7 +3820,7 @@ extern "C" int attn_hip_launch_pack_v(const uint16_t *V, uint16_t *Vp, int Hkv, 
     // (each chunk's base stays 16-byte aligned, since Sk*D is a multiple of 8 on the v16 path).
     constexpr int kMaxZ = 65535;
     for (int h0 = 0; h0 < Hkv; h0 += kMaxZ) {
-        const unsigned nh = (unsigned)min(kMaxZ, Hkv - h0);
+        const unsigned nh = (unsigned)std::min(kMaxZ, Hkv - h0);
         const size_t off = (size_t)h0 * Sk * D;
         constexpr int TK = kPackTK;
         dim3 grid((unsigned)((Sk + TK - 1) / TK), (unsigned)((D + 63) / 64), nh);
