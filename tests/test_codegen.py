@@ -80,3 +80,21 @@ def test_kernels_make_only_the_deliberate_library_call(funcs):
         want = 1 if any(k in name for k in ("attn_prefill_fast_kernel", "attn_prefill_persist_kernel",
                                             "attn_decode_vt_kernel")) else 0
         assert calls == want, (name, calls)
+
+
+def test_split_merge_loads_are_in_flight_together(funcs):
+    """The merge of up to 64 partials is a chain of latencies: its NL column loads per thread are
+    issued back to back, with no wait and no branch between them (branches around the loads cost
+    short merges 1-2 us)."""
+    kernels = {n: ins for n, ins in funcs.items() if "attn_mergew_kernel" in n}
+    assert kernels
+    for name, ins in kernels.items():
+        want = int(re.search(r"attn_mergew_kernelILi(\d+)E", name).group(1))
+        best = run = 0
+        for x in ins:
+            if x.startswith(("s_waitcnt", "s_cbranch", "s_branch", "s_barrier")):
+                run = 0
+            elif x.startswith("global_load_dwordx4"):
+                run += 1
+                best = max(best, run)
+        assert best >= want, (name, best, want)

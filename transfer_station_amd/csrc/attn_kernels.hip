@@ -2790,17 +2790,19 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
 }
 
 // 3 <= nsplit <= kMergeWaveMaxSplit (the prefill key split and decode splits): lp lanes cover a
-// row's columns in 4-float pieces (lp a power of two, 4 lp >= D) and ng groups of them its splits,
-// so a row takes lp * ng threads and a workgroup 256 / (lp ng) rows. Each thread issues its splits'
-// loads (kMergeLoads at a time) before the weights are known; the weights (one wave per row: max and
-// weighted l sum over its lanes) go through LDS, the groups' sums too. With few rows and many
-// splits the launch is latency-bound: one wave per row reading its splits one by one took 7.2 us
-// for 32 rows x 64 splits at D = 128 (8 workgroups); decode over 32768 keys 30.6 -> 26.9 us with this
-// layout, over 777 keys 9.5 -> 8.8.
+// row's columns in 4-float pieces (4 lp >= D; the last piece is the last four floats, so two
+// lanes may write the same columns, with the same values) and ng groups of them its splits, so a row
+// takes lp * ng threads and a workgroup 256 / (lp ng) rows; lp and ng are powers of two (lps, ngs).
+// The launch is a chain of latencies, so everything is in flight at once: the (m, l) of each row's
+// splits (a row per 16 lanes, or per wave past 16 splits), then NL splits' columns per thread
+// without a branch, and only then the weights, which go through LDS, as the groups' sums do. One
+// wave per row reading its splits one by one took 7.2 us for 32 rows x 64 splits at D = 128 (8
+// workgroups); decode over 32768 keys 34.6 -> 30.3 us with this layout. A wave per row for the
+// weights, and branches around the loads, cost short merges 1 to 2 us: 202 rows x 3 splits at
+// D = 32 5.3 us, 10144 rows x 3 at D = 128 8.8.
 constexpr int kMergeWaveMaxSplit = 64;
-constexpr int kMergeLoads = 8;
-// max or sum over the wave's 64 lanes, in every lane, on the VALU.
-template <bool MAX> __device__ __forceinline__ float wave_all(float x) {
+// max or sum over each 16 (all: 64) lanes of the wave, in every lane, on the VALU.
+template <bool MAX> __device__ __forceinline__ float seg_all(float x, bool all) {
     auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
     auto ror = [](float v, auto C) {
         const int u = __builtin_bit_cast(int, v);
@@ -2811,66 +2813,82 @@ template <bool MAX> __device__ __forceinline__ float wave_all(float x) {
     x = op(x, ror(x, std::integral_constant<int, 0x124>{}));
     x = op(x, ror(x, std::integral_constant<int, 0x122>{}));
     x = op(x, ror(x, std::integral_constant<int, 0x121>{}));
-    return MAX ? max_xor32(max_xor16(x)) : sum_xor32(sum_xor16(x));
+    if (all)
+        x = MAX ? max_xor32(max_xor16(x)) : sum_xor32(sum_xor16(x));
+    return x;
 }
+template <int NL>
 __global__ __launch_bounds__(256) void attn_mergew_kernel(const float *__restrict__ pm,
                                                           const float *__restrict__ pl,
                                                           const float *__restrict__ pacc,
                                                           float *__restrict__ O, long rows, int D,
                                                           int nsplit, float c, int rph, int q_off,
-                                                          int Sq, int lp, int ng) {
+                                                          int Sq, int lps, int ngs) {
     __shared__ float wsh[32][kMergeWaveMaxSplit]; // up to 32 rows (lp = 8: D <= 32)
     __shared__ __attribute__((aligned(16))) f32x4 red[256];
     const int tid = wi_id_x(), wv = tid >> 6, lane = tid & 63;
-    const int tpr = lp * ng, rpw = 256 / tpr;
+    const int ng = 1 << ngs, rpw = 256 >> (lps + ngs);
     const long row0 = (long)wg_id_x() * rpw;
-    const int rl = tid / tpr, t = tid - rl * tpr; // the thread's row of the workgroup, lane in it
-    const int g = t / lp, d = 4 * (t - g * lp);
+    const int rl = tid >> (lps + ngs); // the thread's row of the workgroup
+    const int g = (tid >> lps) & (ng - 1), d = 4 * (tid & ((1 << lps) - 1));
     const long row = row0 + rl;
     const bool mine = row < rows && d < D;
-    const float *pr = pacc + (size_t)row * nsplit * D + d;
-    auto piece = [&](int s) -> f32x4 {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f};
-        if (mine && s < nsplit) {
-            const float *p = pr + (size_t)s * D;
-            if (d + 4 <= D) {
-                v = *reinterpret_cast<const f32x4_a4 *>(p);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    if (d + j < D)
-                        v[j] = p[j];
-            }
-        }
-        return v;
+
+    const bool all = nsplit > 16;
+    const int segs = all ? 6 : 4, sl = lane & ((1 << segs) - 1);
+    const int step = 256 >> segs; // rows per pass of the workgroup
+    auto slot_of = [&](int r) {
+        return (size_t)min(row0 + r, rows - 1) * nsplit + min(sl, nsplit - 1);
     };
-    f32x4 x[kMergeLoads];
+    int r = (wv << (6 - segs)) + (lane >> segs);
+    float ms = pm[slot_of(r)], ls = pl[slot_of(r)];
+
+    const float *pr = pacc + (size_t)min(row, rows - 1) * nsplit * D;
+    f32x4 x[NL];
+    auto load = [&](int s0) __attribute__((always_inline)) {
+        const float *p[NL];
 #pragma unroll
-    for (int i = 0; i < kMergeLoads; ++i)
-        x[i] = piece(g + i * ng);
-    for (int r = wv; r < rpw; r += 4) {
-        const bool in = row0 + r < rows && lane < nsplit;
-        const size_t slot = (size_t)(row0 + r) * nsplit + lane;
-        const float ms = in ? pm[slot] : kNegInf;
-        const float ls = in ? pl[slot] : 0.f;
-        const float mx = wave_all<true>(ms);
+        for (int i = 0; i < NL; ++i)
+            p[i] = pr + (size_t)min(s0 + g + i * ng, nsplit - 1) * D;
+        if (D >= 4) {
+#pragma unroll
+            for (int i = 0; i < NL; ++i)
+                x[i] = *reinterpret_cast<const f32x4_a4 *>(p[i] + min(d, D - 4));
+        } else {
+#pragma unroll
+            for (int i = 0; i < NL; ++i)
+                x[i] = f32x4{p[i][0], p[i][D > 1 ? 1 : 0], p[i][D - 1], 0.f};
+        }
+    };
+    load(0);
+    for (;; ms = pm[slot_of(r)], ls = pl[slot_of(r)]) {
+        const bool in = sl < nsplit;
+        const float mx = seg_all<true>(in ? ms : kNegInf, all);
         const float muse = (mx == kNegInf) ? 0.f : mx;
         const float w = in ? fast_exp2((ms - muse) * c) : 0.f;
-        const float lw = wave_all<false>(w * ls);
-        wsh[r][lane] = w * ((lw > 0.f) ? 1.0f / lw : 0.f);
+        const float lw = seg_all<false>(in ? w * ls : 0.f, all);
+        if (r < rpw)
+            wsh[r][sl] = w * ((lw > 0.f) ? 1.0f / lw : 0.f);
+        r += step;
+        if (r - (lane >> segs) >= rpw)
+            break;
     }
     __syncthreads();
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < nsplit; s0 += kMergeLoads * ng) {
+    for (int s0 = 0;;) {
 #pragma unroll
-        for (int i = 0; i < kMergeLoads; ++i) {
+        for (int i = 0; i < NL; ++i) {
             const int s = s0 + g + i * ng;
-            const float a = s < nsplit ? wsh[rl][s] : 0.f;
+            const bool in = s < nsplit;
+            const float a = in ? wsh[rl][s] : 0.f;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                acc[j] += a * x[i][j];
-            x[i] = piece(s + kMergeLoads * ng);
+                acc[j] += a * (in ? x[i][j] : 0.f);
         }
+        s0 += NL * ng;
+        if (s0 >= nsplit)
+            break;
+        load(s0);
     }
     if (ng > 1) {
         red[tid] = acc;
@@ -2878,7 +2896,7 @@ __global__ __launch_bounds__(256) void attn_mergew_kernel(const float *__restric
         if (g != 0)
             return;
         for (int k = 1; k < ng; ++k) {
-            const f32x4 y = red[tid + k * lp];
+            const f32x4 y = red[tid + (k << lps)];
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 acc[j] += y[j];
@@ -2886,13 +2904,13 @@ __global__ __launch_bounds__(256) void attn_mergew_kernel(const float *__restric
     }
     if (!mine)
         return;
-    float *o = O + merge_orow(row, rph, q_off, Sq) * D + d;
-    if (d + 4 <= D) {
-        *reinterpret_cast<f32x4_a4 *>(o) = acc;
+    float *o = O + merge_orow(row, rph, q_off, Sq) * D;
+    if (D >= 4) {
+        *reinterpret_cast<f32x4_a4 *>(o + min(d, D - 4)) = acc;
     } else {
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-            if (d + j < D)
+            if (j < D)
                 o[j] = acc[j];
     }
 }
@@ -3077,21 +3095,24 @@ hipError_t launch_merge(const float *pm, const float *pl, const float *pacc, flo
                                dim3(256), 0, st, pm, pl, pacc, O, rows, D, c, rph, q_off, Sq, lpr);
     }
     else if (nsplit <= kMergeWaveMaxSplit && D <= 256) {
-        int lp = 8;
-        while (4 * lp < D)
-            lp *= 2;
-        // Split groups per row: at most kMergeLoads loads per thread where the workgroup allows, and
-        // more groups (down to two loads per thread) while the grid has fewer threads than the GPU.
-        int ng = 1;
-        while (2 * ng * lp <= 256 && (ng * kMergeLoads < nsplit ||
-                                      (4 * ng <= nsplit && rows * lp * ng < 256L * device_cus())))
-            ng *= 2;
-        const long nwg = (rows + 256 / (lp * ng) - 1) / (256 / (lp * ng));
+        int lps = 3;
+        while ((4 << lps) < D)
+            ++lps;
+        // Split groups per row: at most 8 loads per thread where the workgroup allows, and more
+        // groups (down to two loads per thread) while the grid has fewer threads than the GPU.
+        int ngs = 0;
+        while (ngs + lps < 8 && ((8 << ngs) < nsplit ||
+                                 ((4 << ngs) <= nsplit && rows << (lps + ngs) < 256L * device_cus())))
+            ++ngs;
+        const long rpw = 256 >> (lps + ngs), nwg = (rows + rpw - 1) / rpw;
         if (t_plan)
             plan_note(dim3((unsigned)nwg), dim3(256), "attn_mergew_kernel nsplit=%d", nsplit);
+        else if (nsplit <= 4 << ngs)
+            hipLaunchKernelGGL(attn_mergew_kernel<4>, dim3((unsigned)nwg), dim3(256), 0, st, pm, pl,
+                               pacc, O, rows, D, nsplit, c, rph, q_off, Sq, lps, ngs);
         else
-            hipLaunchKernelGGL(attn_mergew_kernel, dim3((unsigned)nwg), dim3(256), 0, st, pm, pl,
-                               pacc, O, rows, D, nsplit, c, rph, q_off, Sq, lp, ng);
+            hipLaunchKernelGGL(attn_mergew_kernel<8>, dim3((unsigned)nwg), dim3(256), 0, st, pm, pl,
+                               pacc, O, rows, D, nsplit, c, rph, q_off, Sq, lps, ngs);
     } else if (nsplit <= kMergeMaxSplit && D <= 256) {
         if (t_plan)
             plan_note(dim3((unsigned)rows), dim3(256), "attn_merge_kernel nsplit=%d", nsplit);
