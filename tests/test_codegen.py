@@ -98,3 +98,30 @@ def test_split_merge_loads_are_in_flight_together(funcs):
                 run += 1
                 best = max(best, run)
         assert best >= want, (name, best, want)
+
+
+def _decode_kernels(funcs, al):
+    """(DP, V^T, instructions) of the decode kernels of one alignment class (0: unaligned)."""
+    out = []
+    for n, ins in funcs.items():
+        m = re.search(r"attn_decode_kernelILi(\d+)ELb(\d)EL[ib](\d)ELb(\d)E", n)
+        if m and int(m.group(3)) == al:
+            out.append((n, int(m.group(1)), int(m.group(4)), ins))
+    return out
+
+
+def test_unaligned_decode_loads_are_in_flight_together(funcs):
+    """Unaligned rows are read in two steps, so that a tile's K pieces are all in flight before the
+    first is waited for and shifted into place (a shift at the load made decode at small head
+    dims one memory latency per piece)."""
+    kernels = _decode_kernels(funcs, 0)
+    assert kernels
+    for name, dp, vt, ins in kernels:
+        best = run = 0
+        for x in ins:
+            if x.startswith("s_waitcnt") and "vmcnt" in x:
+                run = 0
+            elif x.startswith("global_load_dwordx4"):
+                run += 1
+                best = max(best, run)
+        assert best >= dp // 16, (name, best)  # 2 x DP / 32 K pieces

@@ -159,3 +159,53 @@ def test_decode_groups_and_merges(oracle, case):
     assert ok and nbad == 0, (case, mad, maxref)
     # the same order of sums from V^T, whichever kernel reads it
     assert np.array_equal(O, attend(Q, K, Vt, Hq, Hkv, Sq, Sk, D, causal, 1, 0)), case
+
+
+@pytest.mark.parametrize("case", [
+    # Hq, Hkv, Sq, Sk, D, causal, base offset in elements, what the plan's first kernel holds for
+    # row-major V and for V^T: rows shorter than a piece (", short": of Q, K and V, or of V^T)
+    (4, 2, 1, 300, 1, 0, 0, ", short", ", short"),
+    (4, 2, 2, 5, 1, 1, 0, ", short", ", short"),
+    (4, 2, 1, 3, 2, 0, 1, ", short", ", short"),
+    (8, 2, 3, 777, 7, 1, 0, ", short", ", short"),
+    (64, 64, 1, 2309, 7, 0, 3, ", short", ", short"),
+    (256, 4, 1, 8200, 5, 0, 0, ", short, 2 blocks", ", short, 2 blocks"),
+    (4, 2, 1, 7, 100, 0, 0, "<128, ", ", short"),
+    (4, 2, 2, 7, 200, 1, 0, "<256, ", ", short"),
+    # the staged V^T kernel's limits: D > 32, more than two 128-key steps per part
+    (512, 256, 1, 700, 32, 0, 1, "attn_decode_kernel<64", "attn_decode_kernel<64"),
+    (512, 256, 1, 700, 33, 0, 0, "attn_decode_kernel<64", "attn_decode_vt_kernel<64"),
+    (512, 256, 1, 510, 33, 0, 0, "attn_decode_kernel<64", "attn_decode_kernel<64"),
+    (1024, 512, 1, 257, 121, 0, 0, "attn_decode_kernel<128", "attn_decode_vt_kernel<128"),
+    # pieces at a row's end in both tensors, D % 8 of every kind, at each tile width
+    (8, 2, 1, 1001, 9, 0, 0, "<64, ", "<64, "), (8, 2, 1, 1001, 63, 0, 0, "<64, ", "<64, "),
+    (8, 2, 5, 133, 65, 1, 0, "<128, ", "<128, "), (8, 2, 1, 1023, 127, 0, 1, "<128, ", "<128, "),
+    (8, 2, 1, 1023, 129, 0, 0, "<256, ", "<256, "), (8, 2, 9, 141, 255, 1, 0, "<256, ", "<256, "),
+    (64, 64, 1, 2309, 250, 0, 0, "<256, ", "<256, "), (8, 2, 1, 1000, 256, 0, 1, "<256, ", "<256, "),
+    (8, 2, 1, 1000, 104, 0, 1, "<128, ", "<128, "),
+])
+def test_unaligned_decode(oracle, case):
+    """Decode kernels on tensors without the vector layout, at both sides of the rules between them.
+    Infinite values beyond what a row may see must not reach it: the last key's K row holds some
+    where the causal mask hides it from the first rows."""
+    Hq, Hkv, Sq, Sk, D, causal, off, want, want_t = case
+    print("case", case, flush=True)
+    if ts.device_info()["cus"] == 256 and off == 0:
+        for vt, w in ((0, want), (1, want_t)):
+            name = ts.attn_flash_plan(Hq, Hkv, Sq, Sk, D, causal, v_prepacked=vt)[0][0]
+            if D % 8 or (vt and Sk % 8):
+                assert w in name, (case, vt, name)
+    Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, 313 + D)
+    hide = causal and Sq > 1
+    if hide:
+        K = K.reshape(Hkv, Sk, D).copy()
+        K[:, -1, ::3] = 0x7F80  # only the last query row of a head sees it: not compared
+        K = K.ravel()
+    Vt = np.ascontiguousarray(V.reshape(Hkv, Sk, D).transpose(0, 2, 1)).ravel()
+    rows = np.arange(Sq - 1 if hide else Sq, dtype=np.int32)
+    R = oracle.attn_ref(Q, K, V, Hq, Hkv, Sq, Sk, D, causal, rows, nthreads=8)
+    for vt in (0, 1):
+        O = attend(Q, K, Vt if vt else V, Hq, Hkv, Sq, Sk, D, causal, vt, off)
+        ok, mad, maxref, nbad = oracle.cmp_rows(R, O, Hq, Sq, D, rows)
+        print("   vt=%d err/scale=%.2e nbad=%d" % (vt, mad / maxref, nbad), flush=True)
+        assert ok and nbad == 0, (case, vt, mad, maxref)

@@ -21,7 +21,7 @@
 //                                          back (causal: pairs of a heavy and a light query
 //                                          tile), or (KH) one causal pair of 128-row items on
 //                                          key-tile halves
-//   attn_decode_kernel<DP,CAUSAL,VEC,VT,NTL,NRB> split-K decode for g*Sq <= 64 rows per kv head
+//   attn_decode_kernel<DP,CAUSAL,AL,VT,NTL,NRB> split-K decode for g*Sq <= 64 rows per kv head
 //   attn_decode_vt_kernel<DP,CAUSAL,NTL,UA> the same from V^T, staged in LDS 512 keys at a time
 //   attn_merge{2,w,}_kernel                log-sum-exp merge of split partials (2 splits / up to
 //                                          64 / any, one workgroup per row)
@@ -119,6 +119,13 @@ template <bool NT> __device__ __forceinline__ u32x4 load16_any(const uint16_t *p
               : *reinterpret_cast<const u32x4_a2 *>(p);
 }
 
+// x as a value that the compiler takes for new here: what follows from it is computed where it is
+// used, not hoisted out of the key loop and spilled.
+__device__ __forceinline__ uint32_t opaque(uint32_t x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 // v without its first n (0..8) of eight 16-bit elements, zeros behind.
 __device__ __forceinline__ u32x4 drop_elems(u32x4 v, int n) {
     const int h = (n & 1) * 16;
@@ -131,59 +138,68 @@ __device__ __forceinline__ u32x4 drop_elems(u32x4 v, int n) {
                  n4 || n8 ? 0u : b3};
 }
 
-// Elements [i, i+8) of the n-element row at p, zero-filled past n, at any alignment and without a
-// read outside the row: a chunk that reaches past the row's end is read as its last eight
-// elements and shifted. may (wave-uniform) false: the caller knows that no chunk does. SHORT: the
-// row may have fewer than eight elements.
-template <bool NT = false, bool SHORT = true>
-__device__ __forceinline__ u32x4 load_run8(const uint16_t *p, int i, int n, bool may) {
-    if (!may)
-        return load16_any<NT>(p + i);
-    if (SHORT && n < 8) { // a row shorter than a chunk: element by element, rolled (rare)
-        u32x4 v = zero4();
-#pragma unroll 1
-        for (int j = min(n, i + 8) - 1; j >= i; --j)
-            v = u32x4{(v[0] << 16) | p[j], __builtin_amdgcn_alignbit(v[1], v[0], 16),
-                      __builtin_amdgcn_alignbit(v[2], v[1], 16),
-                      __builtin_amdgcn_alignbit(v[3], v[2], 16)};
-        return v;
-    }
-    const int back = min(max(i + 8 - n, 0), 8);
-    return drop_elems(load16_any<NT>(p + min(i, n - 8)), back);
+// Elements [i, i+8) of the n-element row at p one by one, zero-filled past n: rows of fewer than
+// eight elements. load_rolled does it in a loop: code that hardly any call reaches.
+__device__ __forceinline__ u32x4 load_short(const uint16_t *p, int i, int n) {
+    if (i >= n)
+        return zero4();
+    uint32_t e[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        e[j] = i + j < n ? (uint32_t)p[i + j] : 0u;
+    return u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
 }
 
-// Eight consecutive bf16 of one row, columns [col, col+8), zero-filled past D or when !ok.
-// VEC requires D % 8 == 0 and a 16-byte aligned base, so one 16-byte load covers them; otherwise
-// ce (wave-uniform) bounds the columns of the wave's lanes, so that only a chunk column that
-// reaches past D pays for the shift.
+__device__ __forceinline__ u32x4 load_rolled(const uint16_t *p, int i, int n) {
+    u32x4 v = zero4();
+#pragma unroll 1
+    for (int j = min(n, i + 8) - 1; j >= i; --j)
+        v = u32x4{(v[0] << 16) | p[j], __builtin_amdgcn_alignbit(v[1], v[0], 16),
+                  __builtin_amdgcn_alignbit(v[2], v[1], 16),
+                  __builtin_amdgcn_alignbit(v[3], v[2], 16)};
+    return v;
+}
+
+// Elements [i, i+8) of the n-element row at p (n >= 8), at any alignment and without a read outside
+// the row, in two steps: load_piece reads a piece that reaches past the row's end as its last
+// eight elements, and trim_piece shifts it where it is used, zeros behind (a shift at the load
+// would wait for it before the next piece's load is issued). Pieces past the end are zeros. ie
+// (wave-uniform) bounds the elements of the wave's lanes.
+template <bool NT = false>
+__device__ __forceinline__ u32x4 load_piece(const uint16_t *p, int i, int n, int ie) {
+    if (i >= n)
+        return zero4();
+    if ((n & 7) != 0 && ie > n)
+        return load16_any<NT>(p + min(i, n - 8));
+    return load16_any<NT>(p + i);
+}
+
+__device__ __forceinline__ u32x4 trim_piece(u32x4 v, int i, int n, int ie) {
+    return (n & 7) != 0 && ie > n ? drop_elems(v, (int)opaque(min(max(i + 8 - n, 0), 8))) : v;
+}
+
+// Aligned tensors: eight consecutive bf16 of one row, columns [col, col+8), zero-filled past D or
+// when !ok. D % 8 == 0 and a 16-byte aligned base, so one 16-byte load covers them.
 // NT marks the load non-temporal (data read once: HBM streams such loads ≈ 15% faster).
-template <bool VEC, bool NT = false, bool SHORT = true>
+template <bool NT = false>
 __device__ __forceinline__ u32x4 load_row8(const uint16_t *base, size_t row, int col, int D,
-                                           bool ok, int ce = 0x7fffffff) {
+                                           bool ok) {
     if (!ok || col >= D)
         return zero4();
-    const uint16_t *p = base + row * (size_t)D;
-    if (!VEC)
-        return load_run8<NT, SHORT>(p, col, D, (D & 7) != 0 && ce > D);
-    p += col;
+    const uint16_t *p = base + row * (size_t)D + col;
     return NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p))
               : *reinterpret_cast<const u32x4 *>(p);
 }
 
-// Eight consecutive keys [key, key+8) of row d of a V^T head ([D][Sk], row stride Sk), zero-filled
-// at d >= D or key >= klim. VEC requires Sk % 8 == 0 (with key % 8 == 0 and klim % 8 == 0 a chunk
-// is then wholly inside or wholly outside) and a 16-byte aligned base; otherwise ke
-// (wave-uniform) bounds the keys of the wave's lanes, and klim is a multiple of 8 above key or Sk
-// (the row's end), as for the keys of a tile.
-template <bool VEC, bool NT = false>
+// Aligned tensors: eight consecutive keys [key, key+8) of row d of a V^T head ([D][Sk], row stride
+// Sk), zero-filled at d >= D or key >= klim. Sk % 8 == 0 and a 16-byte aligned base (with
+// key % 8 == 0 and klim % 8 == 0 a chunk is then wholly inside or wholly outside).
+template <bool NT = false>
 __device__ __forceinline__ u32x4 load_vt8(const uint16_t *base, int d, int key, int Sk, int D,
-                                          int klim, int ke = 0x7fffffff) {
+                                          int klim) {
     if (d >= D || key >= klim)
         return zero4();
-    const uint16_t *p = base + (size_t)d * Sk;
-    if (!VEC)
-        return load_run8<NT>(p, key, klim, ke > klim);
-    p += key;
+    const uint16_t *p = base + (size_t)d * Sk + key;
     return NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p))
               : *reinterpret_cast<const u32x4 *>(p);
 }
@@ -560,9 +576,17 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         }
     } else {
 #pragma unroll
-        for (int kk = 0; kk < DP / 16; ++kk)
-            qb[kk] = as_bf16x8(load_row8<UA == 0, false, UA == 2>(Q, qrow, kk * 16 + hi * 8, D,
-                                                                  rvalid, kk * 16 + 16));
+        for (int kk = 0; kk < DP / 16; ++kk) {
+            const int col = kk * 16 + hi * 8;
+            u32x4 v = zero4();
+            if constexpr (UA == 0)
+                v = load_row8(Q, qrow, col, D, rvalid);
+            else if (rvalid)
+                v = UA == 2 ? load_rolled(Q + qrow * D, col, D)
+                            : trim_piece(load_piece(Q + qrow * D, col, D, kk * 16 + 16), col, D,
+                                         kk * 16 + 16);
+            qb[kk] = as_bf16x8(v);
+        }
     }
     // Q stays in flight while the first tile's DMA is issued; one wait before the loop covers
     // both (below).
@@ -649,8 +673,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     // UA: this wave's pieces of a K (or V) tile into registers, and from there into LDS. Every load
     // stays inside its row: a piece that reaches past the row's end is read as the row's last
     // eight elements and shifted where it is put into LDS (shifting it at the load would wait for
-    // it). One packed offset per piece is kept and made opaque where it is used: what follows
-    // from it would otherwise be hoisted out of the key loop and spilled.
+    // it). One packed offset per piece is kept and made opaque where it is used.
     constexpr int UPW = UA ? PW : 1;
     constexpr bool TINY = UA == 2; // rows of fewer than eight elements: element by element
     u32x4 gk[UPW], gv[UPW];
@@ -676,10 +699,6 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         ktail = __builtin_amdgcn_readfirstlane(ktail);
         vtail = __builtin_amdgcn_readfirstlane(vtail);
     }
-    auto opaque = [](uint32_t x) __attribute__((always_inline)) {
-        asm volatile("" : "+v"(x));
-        return x;
-    };
     auto ua_rows = [&](const uint16_t *H, int kt, const uint32_t *pk, u32x4 *gr)
         __attribute__((always_inline)) {
         const uint16_t *T = H + (size_t)kt * KT * D;
@@ -693,7 +712,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
                     const int r = (int)(x >> 6), col = (int)(x & 63);
                     gr[k] = zero4();
                     if (kt * KT + r < Sk && col < D)
-                        gr[k] = load_run8(T + r * D, col, D, true);
+                        gr[k] = load_rolled(T + r * D, col, D);
                 } else { // rows past the last key read its last elements
                     gr[k] = load16_any<false>(T + min(x >> 4, last - 8));
                 }
@@ -730,7 +749,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
                 key += kt * KT;
                 const uint16_t *row = Vh + (size_t)e * Sk;
                 if (TINY || Sk < 8)
-                    gv[k] = key < Sk ? load_run8(row, key, Sk, true) : zero4();
+                    gv[k] = key < Sk ? load_rolled(row, key, Sk) : zero4();
                 else
                     gv[k] = load16_any<false>(row + min(key, Sk - 8));
             }
@@ -2240,6 +2259,11 @@ __device__ __forceinline__ void decode_merge(const float *om, const float (*red_
 // then loaded from global memory straight into its register layout, like K, with no LDS tile.
 // NTL: K and V are loaded non-temporally (decode_nt_loads decides).
 // ------------------------------------------------------------------------------------------
+// AL: 1 tensors with the 16-byte vector layout; 0 without, read in pieces (load_piece, trim_piece);
+// 2 rows shorter than a piece (D < 8, or V^T of fewer than 8 keys), read element by element. What
+// bounds AL = 0 at small head dims is latency, so no piece is shifted before all of a tile's are in
+// flight (shifted at the load -> so): 256 kv heads x 300 keys at D = 14 13.6 -> 8.7 us from V^T, 8 kv
+// heads x 777 keys at D = 100 10.4 -> 8.8.
 // NRB: the row blocks one workgroup serves (rb counts groups of NRB); each K/V fragment is then read
 // once for all of them. Each row's arithmetic is that of NRB = 1. Two blocks for three or four of a
 // kv head (launch_decode_d): 64 rows over 4001 keys, 32 kv heads 28.6 -> 23.2 us, 128 kv heads over
@@ -2249,7 +2273,7 @@ __device__ __forceinline__ void decode_merge(const float *om, const float (*red_
 // (+5 to +12%, the registers take a wave per SIMD).
 // Two waves per SIMD are asked for; the 138 registers at D = 128 allow three (172 with no bound:
 // c2 162.4 -> 160 us, D = 256 with 8 kv heads 18.7 -> 14.9).
-template <int DP, bool CAUSAL, bool VEC, bool VT, bool NTL, int NRB>
+template <int DP, bool CAUSAL, int AL, bool VT, bool NTL, int NRB>
 __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     const uint16_t *__restrict__ V, float *__restrict__ O, float *__restrict__ pm,
@@ -2282,10 +2306,17 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
     const int r16 = lane & 15, grp = lane >> 4;
     const int k0 = sp * kps, k1 = min(k0 + kps, Sk);
     const int row0 = 16 * NRB * rb;
+    constexpr bool VEC = AL == 1;
 
     const uint16_t *Kh = K + (size_t)u * Sk * D;
     const uint16_t *Vh = V + (size_t)u * Sk * D;
 
+    auto piece = [](const uint16_t *p, int i, int n, int ie) __attribute__((always_inline)) {
+        return AL == 2 ? load_short(p, i, n) : load_piece<NTL>(p, i, n, ie);
+    };
+    auto trim = [](u32x4 v, int i, int n, int ie) __attribute__((always_inline)) {
+        return AL == 0 ? trim_piece(v, i, n, ie) : v;
+    };
     bf16x8 qb[NRB][DP / 32];
     int lim[NRB];
     float m_run[NRB], l_run[NRB];
@@ -2295,11 +2326,16 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
         const int row = row0 + 16 * b + r16;
         const bool rvalid = row < M;
         const int gi = rvalid ? row / Sq : 0, qi = rvalid ? row % Sq : 0;
+        const size_t qrow = (size_t)(u * g + gi) * Sq + qi;
+        u32x4 qr[DP / 32];
 #pragma unroll
         for (int kk = 0; kk < DP / 32; ++kk)
-            qb[b][kk] =
-                as_bf16x8(load_row8<VEC>(Q + (size_t)(u * g + gi) * Sq * D, (size_t)qi,
-                                         kk * 32 + grp * 8, D, rvalid, kk * 32 + 32));
+            qr[kk] = VEC ? load_row8(Q, qrow, kk * 32 + grp * 8, D, rvalid)
+                         : piece(Q + qrow * D, kk * 32 + grp * 8, D, kk * 32 + 32);
+#pragma unroll
+        for (int kk = 0; kk < DP / 32; ++kk)
+            qb[b][kk] = as_bf16x8(VEC || rvalid ? trim(qr[kk], kk * 32 + grp * 8, D, kk * 32 + 32)
+                                                : zero4());
         lim[b] = CAUSAL ? min(Sk - 1, Sk - Sq + qi) : Sk - 1;
         m_run[b] = kNegInf;
         l_run[b] = 0.f;
@@ -2322,27 +2358,64 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
         u32x4 k[2][DP / 32];
         u32x4 v[VT ? DP / 16 : VNCH];
     };
-    auto load = [&](int tb, frags &f) __attribute__((always_inline)) {
+    // Unaligned pieces (AL != 1) of keys past k1 are those of key k1 - 1: their scores are masked,
+    // their V rows zeroed (trim_v).
+    auto load_k = [&](int tb, frags &f) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const int key = tb + 8 * (r16 >> 2) + 4 * t + (r16 & 3);
 #pragma unroll
             for (int kk = 0; kk < DP / 32; ++kk)
-                f.k[t][kk] = load_row8<VEC, NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1,
-                                                 kk * 32 + 32);
+                f.k[t][kk] = VEC ? load_row8<NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1)
+                                 : piece(Kh + (size_t)min(key, k1 - 1) * D, kk * 32 + grp * 8, D,
+                                         kk * 32 + 32);
         }
-        if (VT) {
+    };
+    auto load_v = [&](int tb, frags &f) __attribute__((always_inline)) {
+        if constexpr (VT) {
             // lane: d row 16db + r16, keys tb + 8grp .. +7 (the k index of pk below).
+            const int key = tb + 8 * grp;
 #pragma unroll
-            for (int db = 0; db < DP / 16; ++db)
-                f.v[db] =
-                    load_vt8<VEC, NTL>(Vh, db * 16 + r16, tb + 8 * grp, Sk, D, k1, tb + 32);
+            for (int db = 0; db < DP / 16; ++db) {
+                const int d = db * 16 + (VEC ? r16 : (int)opaque(r16));
+                if (VEC) {
+                    f.v[db] = load_vt8<NTL>(Vh, d, key, Sk, D, k1);
+                } else {
+                    f.v[db] = zero4();
+                    if (d < D) // rows past D are never stored
+                        f.v[db] = piece(Vh + (size_t)d * Sk, key, k1, tb + 32);
+                }
+            }
         } else {
 #pragma unroll
             for (int r = 0; r < VNCH; ++r) {
                 const int cidx = lane + 64 * r;
-                const int row = cidx / (DP / 8), col = (cidx % (DP / 8)) * 8;
-                f.v[r] = load_row8<VEC, NTL>(Vh, (size_t)(tb + row), col, D, tb + row < k1);
+                const int row = tb + cidx / (DP / 8), col = (cidx % (DP / 8)) * 8;
+                f.v[r] = VEC ? load_row8<NTL>(Vh, (size_t)row, col, D, row < k1)
+                             : piece(Vh + (size_t)min(row, k1 - 1) * D, col, D, DP);
+            }
+        }
+    };
+    auto trim_k = [&](frags &f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int kk = 0; kk < DP / 32; ++kk)
+                f.k[t][kk] = trim(f.k[t][kk], kk * 32 + grp * 8, D, kk * 32 + 32);
+    };
+    auto trim_v = [&](int tb, frags &f) __attribute__((always_inline)) {
+        if constexpr (VT) {
+#pragma unroll
+            for (int db = 0; db < DP / 16; ++db)
+                f.v[db] = trim(f.v[db], tb + 8 * grp, k1, tb + 32);
+        } else {
+#pragma unroll
+            for (int r = 0; r < VNCH; ++r) {
+                const int cidx = lane + 64 * r;
+                const int row = tb + cidx / (DP / 8), col = (cidx % (DP / 8)) * 8;
+                f.v[r] = trim(f.v[r], col, D, DP);
+                if (!VEC && tb + 32 > k1)
+                    f.v[r] = row < k1 ? f.v[r] : zero4();
             }
         }
     };
@@ -2427,7 +2500,10 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
         if (tb >= k1)
             continue;
         frags f;
-        load(tb, f);
+        load_k(tb, f);
+        load_v(tb, f);
+        trim_k(f);
+        trim_v(tb, f);
         put_v(f);
         compute(tb, f);
     }
@@ -2506,11 +2582,17 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
     const uint16_t *Kh = K + (size_t)u * Sk * D;
 
     bf16x8 qb[DP / 32];
+    const size_t qrow = (size_t)h * Sq + qi;
+    u32x4 qr[DP / 32];
 #pragma unroll
     for (int kk = 0; kk < DP / 32; ++kk)
-        qb[kk] = as_bf16x8(
-            load_row8<!UA>(Q + (size_t)h * Sq * D, (size_t)qi, kk * 32 + grp * 8, D, rvalid,
-                           kk * 32 + 32));
+        qr[kk] = UA ? load_piece(Q + qrow * D, kk * 32 + grp * 8, D, kk * 32 + 32)
+                    : load_row8(Q, qrow, kk * 32 + grp * 8, D, rvalid);
+#pragma unroll
+    for (int kk = 0; kk < DP / 32; ++kk)
+        qb[kk] = as_bf16x8(!UA      ? qr[kk]
+                           : rvalid ? trim_piece(qr[kk], kk * 32 + grp * 8, D, kk * 32 + 32)
+                                    : zero4());
     const int lim = CAUSAL ? min(Sk - 1, Sk - Sq + qi) : Sk - 1;
 
     float m_run = kNegInf, l_run = 0.f;
@@ -2583,17 +2665,30 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
             const int key = tb + 8 * (r16 >> 2) + 4 * t + (r16 & 3);
 #pragma unroll
             for (int kk = 0; kk < DP / 32; ++kk)
-                dst[t][kk] = load_row8<!UA, NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1,
-                                                 kk * 32 + 32);
+                dst[t][kk] =
+                    UA ? load_piece<NTL>(Kh + (size_t)min(key, k1 - 1) * D, kk * 32 + grp * 8, D,
+                                         kk * 32 + 32)
+                       : load_row8<NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1);
         }
+    };
+    // src, as load_k put it there, into ka.
+    auto take_k = [&](const u32x4 (&src)[2][DP / 32]) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int kk = 0; kk < DP / 32; ++kk)
+                ka[t][kk] = UA ? trim_piece(src[t][kk], kk * 32 + grp * 8, D, kk * 32 + 32)
+                               : src[t][kk];
     };
 
     bf16x8 pkp[4], pkc[4]; // softmax weights of the previous / current group's steps
     float alp[4], alc[4];  // their rescale factors
     int livep = 0, livec = 0; // bit st: step st of the previous / current group was scored
     int buf = 0;
-    if (ngr > 0)
-        load_k(k0 + step_of(0) * 128 + w * 32, ka);
+    if (ngr > 0) {
+        load_k(k0 + step_of(0) * 128 + w * 32, kn);
+        take_k(kn);
+    }
     for (int j = 0; j <= ngr; ++j) {
         const bool cur = j < ngr;
         const int nsub = cur ? min(4, nsteps - 4 * j) : 0;
@@ -2675,13 +2770,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
             }
             // The next step's K fragments (waiting for them here leaves the loads in flight
             // under both halves of the interval).
-            if (tbn >= 0) {
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int kk = 0; kk < DP / 32; ++kk)
-                        ka[t][kk] = kn[t][kk];
-            }
+            if (tbn >= 0)
+                take_k(kn);
             if (UA && (i < 3 ? j > 0 : cur))
                 put_tile(i < 3 ? j - 1 : j, buf ^ 1);
             buf ^= 1;
@@ -2989,7 +3079,9 @@ __global__ __launch_bounds__(256) void attn_pack_v16_kernel(const uint16_t *__re
         if (k < Sk && d < D)
             v = VEC ? __builtin_nontemporal_load(
                           reinterpret_cast<const u32x4 *>(src + (size_t)k * D + d))
-                    : load_run8<true>(src + (size_t)k * D, d, D, d0 + TD > D);
+                    : D < 8 ? load_short(src + (size_t)k * D, d, D)
+                            : trim_piece(load_piece<true>(src + (size_t)k * D, d, D, d0 + TD), d, D,
+                                         d0 + TD);
         *reinterpret_cast<u32x4 *>(&tile[row * TD + ((ch ^ (row >> 3)) & 7) * 8]) = v;
     }
     __syncthreads();
@@ -3678,10 +3770,13 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
     // attn_decode_kernel straight from V^T 8.2; over 777 keys 14.2 and 10.0; two steps and up it is
     // the faster one, 64 kv heads over 3001 keys 24.0 and 28.0). Its DMA offsets are 32-bit: a head's
     // aligned V^T must stay below 2 GiB. Grouped row blocks read V^T once straight from memory (32 kv
-    // heads, 64 rows over 4000 keys: staged per block 33, this 25.5).
+    // heads, 64 rows over 4000 keys: staged per block 33, this 25.5). Unaligned V^T passes through
+    // registers on its way to LDS, padding rows too, so there the staged kernel needs D > 32 and more
+    // than two steps: against attn_decode_kernel, 128 kv heads x 4001 keys at D = 100 46.4 and 54.9
+    // us, at D = 20 1.15-1.2 times its time, with two steps at any D 1.0 to 1.4 times.
     if constexpr (DP <= 128)
         if (vt && blocks == 1 && kps > ATTN_DECODE_MIN_KEYS && decode_vt_staged() &&
-            (vec ? (long)D * Sk * 2 < 0x7fffffffL : Sk >= 8))
+            (vec ? (long)D * Sk * 2 < 0x7fffffffL : D > 32 && kps > 2 * ATTN_DECODE_MIN_KEYS))
             return with_flag(causal != 0, [&](auto CA) {
                 return with_flag(ntl, [&](auto NT) {
                     return with_flag(vec == 0, [&](auto UAF) {
@@ -3704,24 +3799,30 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
         constexpr int NRB = decltype(NB)::value;
         const int ng = (nrb + NRB - 1) / NRB; // row block groups
         const long n = (long)Hkv * nsplit * ng;
+        auto launch = [&](auto CA, auto ALF, auto VTF, auto NT) {
+            constexpr bool kC = decltype(CA)::value, kT = decltype(VTF)::value,
+                           kN = decltype(NT)::value;
+            constexpr int kA = decltype(ALF)::value;
+            if (t_plan)
+                plan_note(dim3((unsigned)n), dim3(256),
+                          "attn_decode_kernel<%d, %s, %s, %s, %s%s%s> nsplit=%d nrb=%d", DP,
+                          tf(kC), tf(kA == 1), tf(kT), tf(kN), kA == 2 ? ", short" : "",
+                          NRB == 2 ? ", 2 blocks" : "", nsplit, nrb);
+            else
+                hipLaunchKernelGGL((attn_decode_kernel<DP, kC, kA, kT, kN, NRB>),
+                                   dim3((unsigned)n), dim3(256), 0, st, Q, K, V, O, pm, pl, pacc,
+                                   Hq, Hkv, Sq, Sk, D, c, nsplit, kps, ng);
+            return hipGetLastError();
+        };
         return with_flag(causal != 0, [&](auto CA) {
-            return with_flag(vec != 0, [&](auto VE) {
-                return with_flag(vt != 0, [&](auto VTF) {
-                    return with_flag(ntl, [&](auto NT) {
-                        constexpr bool kC = decltype(CA)::value, kE = decltype(VE)::value,
-                                       kT = decltype(VTF)::value, kN = decltype(NT)::value;
-                        if (t_plan)
-                            plan_note(dim3((unsigned)n), dim3(256),
-                                      "attn_decode_kernel<%d, %s, %s, %s, %s%s> nsplit=%d nrb=%d",
-                                      DP, tf(kC), tf(kE), tf(kT), tf(kN),
-                                      NRB == 2 ? ", 2 blocks" : "",
-                                      nsplit, nrb);
-                        else
-                            hipLaunchKernelGGL((attn_decode_kernel<DP, kC, kE, kT, kN, NRB>),
-                                               dim3((unsigned)n), dim3(256), 0, st, Q, K, V, O, pm,
-                                               pl, pacc, Hq, Hkv, Sq, Sk, D, c, nsplit, kps, ng);
-                        return hipGetLastError();
-                    });
+            return with_flag(vt != 0, [&](auto VTF) {
+                // Rows shorter than a piece: of Q, K and V (D < 8, so DP = 64) or of V^T.
+                if constexpr (DP == 64 || decltype(VTF)::value)
+                    if (!vec && (D < 8 || (vt && Sk < 8)))
+                        return launch(CA, std::integral_constant<int, 2>{}, VTF, std::false_type{});
+                return with_flag(ntl, [&](auto NT) {
+                    return vec ? launch(CA, std::integral_constant<int, 1>{}, VTF, NT)
+                               : launch(CA, std::integral_constant<int, 0>{}, VTF, NT);
                 });
             });
         });
