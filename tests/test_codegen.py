@@ -12,6 +12,7 @@ import os
 import re
 import shutil
 import subprocess
+import tempfile
 
 import pytest
 
@@ -125,3 +126,29 @@ def test_unaligned_decode_loads_are_in_flight_together(funcs):
                 run += 1
                 best = max(best, run)
         assert best >= dp // 16, (name, best)  # 2 x DP / 32 K pieces
+
+
+def test_decode_kernels_do_not_spill():
+    """attn_decode_kernel asks for two waves per SIMD, which leaves 256 registers: no instance may
+    pay for that with spills on every tile (unaligned rows past D = 128 once spilled 90-112, up to
+    1.8 times the time without)."""
+    readelf = os.path.join(ROCM, "llvm", "bin", "llvm-readelf")
+    if not os.path.exists(_build.lib_path()):
+        pytest.skip("library not built")
+    if not os.access(readelf, os.X_OK) or not os.access(OBJDUMP, os.X_OK):
+        pytest.skip("llvm tools not found under %s" % ROCM)
+    with tempfile.TemporaryDirectory() as tmp:
+        copy = os.path.join(tmp, "lib.so")
+        shutil.copy(_build.lib_path(), copy)
+        subprocess.run([OBJDUMP, "--offloading", copy], cwd=tmp, check=True,
+                       stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+        obj = [f for f in os.listdir(tmp) if f.endswith("gfx950")]
+        assert len(obj) == 1, obj
+        notes = subprocess.run([readelf, "--notes", os.path.join(tmp, obj[0])], check=True,
+                               stdout=subprocess.PIPE, universal_newlines=True).stdout
+    spills = {m.group(1): int(m.group(2)) for m in re.finditer(
+        r"\.symbol: +'?(\S*?attn_decode_kernel\S*?)\.kd'?\n(?:.*\n)*? +\.vgpr_spill_count: +(\d+)",
+        notes)}
+    assert len(spills) >= 40, len(spills)
+    bad = {n: c for n, c in spills.items() if c}
+    assert not bad, bad

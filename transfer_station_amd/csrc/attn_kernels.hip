@@ -2274,7 +2274,7 @@ __device__ __forceinline__ void decode_merge(const float *om, const float (*red_
 // Two waves per SIMD are asked for; the 138 registers at D = 128 allow three (172 with no bound:
 // c2 162.4 -> 160 us, D = 256 with 8 kv heads 18.7 -> 14.9).
 template <int DP, bool CAUSAL, int AL, bool VT, bool NTL, int NRB>
-__global__ __launch_bounds__(256, 2) void attn_decode_kernel(
+__global__ __launch_bounds__(256, DP == 256 && VT && AL == 2 ? 1 : 2) void attn_decode_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     const uint16_t *__restrict__ V, float *__restrict__ O, float *__restrict__ pm,
     float *__restrict__ pl, float *__restrict__ pacc, int Hq, int Hkv, int Sq, int Sk, int D,
@@ -2358,6 +2358,12 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
         u32x4 k[2][DP / 32];
         u32x4 v[VT ? DP / 16 : VNCH];
     };
+    // At DP = 256 K, V, Q and O of a tile do not fit the 256 registers of two waves per SIMD unless both
+    // tensors are aligned and V is row-major: there V is loaded once Q.K^T has freed K's registers.
+    // Spilling instead (12 registers aligned, 90-112 unaligned) -> so, 64 kv heads: 16000 keys at
+    // D = 256 from V^T 250 -> 227 us, 4000 keys at D = 131 from V^T 67 -> 39 (one wave per SIMD, no
+    // spills, V loaded with K: 54).
+    constexpr bool kLate = DP == 256 && (VT || !VEC);
     // Unaligned pieces (AL != 1) of keys past k1 are those of key k1 - 1: their scores are masked,
     // their V rows zeroed (trim_v).
     auto load_k = [&](int tb, frags &f) __attribute__((always_inline)) {
@@ -2431,7 +2437,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
             }
         }
     };
-    auto compute = [&](int tb, const frags &f) __attribute__((always_inline)) {
+    auto compute = [&](int tb, frags &f) __attribute__((always_inline)) {
         bf16x8 pk[NRB];
 #pragma unroll
         for (int b = 0; b < NRB; ++b) {
@@ -2443,6 +2449,10 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
                 for (int kk = 0; kk < DP / 32; ++kk)
                     s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(f.k[t][kk]),
                                                                    qb[b][kk], s[t], 0, 0, 0);
+            }
+            if (kLate) { // NRB == 1
+                __builtin_amdgcn_sched_barrier(0);
+                load_v(tb, f);
             }
             // Register (t, i) of this lane holds key tb + 8grp + 4t + i for row r16.
             float mx = kNegInf;
@@ -2475,6 +2485,10 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
             for (int db = 0; db < DP / 16; ++db)
                 o[b][db] *= alpha;
         }
+        if (kLate) {
+            trim_v(tb, f);
+            put_v(f);
+        }
         if (!VT)
             lds_wave_fence(); // this tile's V is in LDS before the transposed reads
         // rows of this lane's reads: 8grp + r16/4 and 4 on, in row-octet grp
@@ -2501,10 +2515,13 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
             continue;
         frags f;
         load_k(tb, f);
-        load_v(tb, f);
+        if (!kLate)
+            load_v(tb, f);
         trim_k(f);
-        trim_v(tb, f);
-        put_v(f);
+        if (!kLate) {
+            trim_v(tb, f);
+            put_v(f);
+        }
         compute(tb, f);
     }
 #pragma unroll
