@@ -152,3 +152,14 @@ def test_decode_kernels_do_not_spill():
     assert len(spills) >= 40, len(spills)
     bad = {n: c for n, c in spills.items() if c}
     assert not bad, bad
+
+
+def test_short_row_prefill_loads_rows_whole(funcs):
+    """Head dims below 8: a K or V row is one 16-byte load (element by element, in a loop that waited
+    for each, these prefills took up to 1.5 times as long)."""
+    kernels = {n: ins for n, ins in funcs.items()
+               if re.search(r"attn_prefill_fast_kernelILi64ELi128ELi4E.*Li2EE", n)}
+    assert len(kernels) == 4, sorted(kernels)
+    for name, ins in kernels.items():
+        # K, and V or V^T: four pieces per thread each, at the first tile and in the loop
+        assert sum(x.startswith("global_load_dwordx4") for x in ins) >= 16, name

@@ -209,3 +209,26 @@ def test_unaligned_decode(oracle, case):
         ok, mad, maxref, nbad = oracle.cmp_rows(R, O, Hq, Sq, D, rows)
         print("   vt=%d err/scale=%.2e nbad=%d" % (vt, mad / maxref, nbad), flush=True)
         assert ok and nbad == 0, (case, vt, mad, maxref)
+
+
+@pytest.mark.parametrize("case", [
+    # Hq, Hkv, Sq, Sk, D, causal, base offset: prefill of rows shorter than a piece
+    (2, 1, 100, 1, 1, 0, 0), (2, 1, 100, 7, 1, 1, 0), (2, 1, 100, 8, 1, 0, 1),  # heads of 1-8 elements
+    (2, 2, 70, 2, 3, 0, 0), (2, 2, 70, 3, 3, 1, 1), (2, 1, 70, 1, 7, 0, 0), (2, 1, 70, 2, 5, 1, 0),
+    (3, 3, 130, 129, 1, 0, 0), (3, 3, 130, 130, 3, 1, 0), (3, 3, 130, 257, 7, 0, 3),  # short last tiles
+    (4, 2, 200, 128, 5, 0, 0), (4, 2, 200, 263, 2, 1, 1), (64, 64, 65, 385, 6, 1, 0),
+    (8, 4, 101, 1801, 7, 0, 0), (8, 4, 300, 900, 3, 1, 0),  # key splits
+    (32, 8, 20, 333, 4, 1, 1), (600, 600, 140, 300, 5, 0, 0),
+])
+def test_short_row_prefill(oracle, case):
+    Hq, Hkv, Sq, Sk, D, causal, off = case
+    print("case", case, flush=True)
+    Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, 17 + D)
+    Vt = np.ascontiguousarray(V.reshape(Hkv, Sk, D).transpose(0, 2, 1)).ravel()
+    rows = oracle.ref_rowset(Sq, 16)
+    R = oracle.attn_ref(Q, K, V, Hq, Hkv, Sq, Sk, D, causal, rows, nthreads=8)
+    for vt in (0, 1):
+        O = attend(Q, K, Vt if vt else V, Hq, Hkv, Sq, Sk, D, causal, vt, off)
+        ok, mad, maxref, nbad = oracle.cmp_rows(R, O, Hq, Sq, D, rows)
+        print("   vt=%d err/scale=%.2e nbad=%d" % (vt, mad / maxref, nbad), flush=True)
+        assert ok and nbad == 0, (case, vt, mad, maxref)

@@ -160,6 +160,14 @@ __device__ __forceinline__ u32x4 load_rolled(const uint16_t *p, int i, int n) {
     return v;
 }
 
+// The first m (1..7) of eight 16-bit elements, zeros behind.
+__device__ __forceinline__ u32x4 keep_elems(u32x4 v, int m) {
+    auto w = [&](uint32_t x, int j) {
+        return m >= 2 * j + 2 ? x : m == 2 * j + 1 ? x & 0xffffu : 0u;
+    };
+    return u32x4{w(v[0], 0), w(v[1], 1), w(v[2], 2), w(v[3], 3)};
+}
+
 // Elements [i, i+8) of the n-element row at p (n >= 8), at any alignment and without a read outside
 // the row, in two steps: load_piece reads a piece that reaches past the row's end as its last
 // eight elements, and trim_piece shifts it where it is used, zeros behind (a shift at the load
@@ -582,7 +590,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
             if constexpr (UA == 0)
                 v = load_row8(Q, qrow, col, D, rvalid);
             else if (rvalid)
-                v = UA == 2 ? load_rolled(Q + qrow * D, col, D)
+                v = UA == 2 ? load_short(Q + qrow * D, col, D)
                             : trim_piece(load_piece(Q + qrow * D, col, D, kk * 16 + 16), col, D,
                                          kk * 16 + 16);
             qb[kk] = as_bf16x8(v);
@@ -675,7 +683,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     // eight elements and shifted where it is put into LDS (shifting it at the load would wait for
     // it). One packed offset per piece is kept and made opaque where it is used.
     constexpr int UPW = UA ? PW : 1;
-    constexpr bool TINY = UA == 2; // rows of fewer than eight elements: element by element
+    constexpr bool TINY = UA == 2; // rows of fewer than eight elements
     u32x4 gk[UPW], gv[UPW];
     const uint16_t *Kh = K + (size_t)u * Sk * D, *Vh = V + (size_t)u * Sk * D;
     // Row-major piece k: (element offset of its eight elements in the tile) * 16 + how many of
@@ -699,6 +707,11 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         ktail = __builtin_amdgcn_readfirstlane(ktail);
         vtail = __builtin_amdgcn_readfirstlane(vtail);
     }
+    // TINY: a row is one piece, the rows after it behind it; the head's last rows are read with its
+    // last eight elements, at this offset from tile kt's first (below 0 where that tile is shorter).
+    auto tiny_last = [&](int kt) {
+        return (int)min((long)(Sk - kt * KT) * D, (long)KT * 8) - 8;
+    };
     auto ua_rows = [&](const uint16_t *H, int kt, const uint32_t *pk, u32x4 *gr)
         __attribute__((always_inline)) {
         const uint16_t *T = H + (size_t)kt * KT * D;
@@ -709,10 +722,11 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
             if (NI % NW == 0 || k < nblk_w) {
                 const uint32_t x = opaque(pk[k]);
                 if constexpr (TINY) {
-                    const int r = (int)(x >> 6), col = (int)(x & 63);
+                    const int r = (int)(x >> 6);
                     gr[k] = zero4();
-                    if (kt * KT + r < Sk && col < D)
-                        gr[k] = load_rolled(T + r * D, col, D);
+                    if ((x & 63) == 0 && kt * KT + r < Sk)
+                        gr[k] = (long)Sk * D < 8 ? load_rolled(T + r * D, 0, D)
+                                                 : load16_any<false>(T + min(r * D, tiny_last(kt)));
                 } else { // rows past the last key read its last elements
                     gr[k] = load16_any<false>(T + min(x >> 4, last - 8));
                 }
@@ -726,6 +740,10 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
         for (int k = 0; k < PW; ++k)
             if (NI % NW == 0 || k < nblk_w) {
                 u32x4 v = gr[k];
+                if (TINY && (long)Sk * D >= 8) {
+                    const int at = (int)(opaque(pk[k]) >> 6) * D;
+                    v = keep_elems(drop_elems(v, min(8, max(0, at - tiny_last(kt)))), D);
+                }
                 if (!TINY && (tail >> k & 1))
                     v = drop_elems(v, (int)(opaque(pk[k]) & 15));
                 if (edge)
@@ -748,14 +766,14 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
                 vt_piece(k, e, key);
                 key += kt * KT;
                 const uint16_t *row = Vh + (size_t)e * Sk;
-                if (TINY || Sk < 8)
-                    gv[k] = key < Sk ? load_rolled(row, key, Sk) : zero4();
+                if (Sk < 8)
+                    gv[k] = load_rolled(row, key, Sk);
                 else
                     gv[k] = load16_any<false>(row + min(key, Sk - 8));
             }
     };
     auto put_vt = [&](uint16_t *tile, int kt) __attribute__((always_inline)) {
-        const bool edge = !TINY && Sk >= 8 && kt * KT + KT > Sk;
+        const bool edge = Sk >= 8 && kt * KT + KT > Sk;
 #pragma unroll
         for (int k = 0; k < PW; ++k)
             if (NI % NW == 0 || k < nblk_w) {
@@ -1422,7 +1440,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     }
     const float inv = (lt > 0.f) ? 1.0f / lt : 0.f;
     bool staged = false;
-    if constexpr (KT >= 16 * NW && DP <= 128) {
+    if constexpr (KT >= 16 * NW && DP <= 128 && UA != 2) { // rows of D < 8 fit one 32-byte piece
         if (!pack) {
             staged = true;
             // O leaves through LDS. Each wave writes its rows there in the accumulator layout (a
