@@ -135,20 +135,32 @@ def test_wide_head_dims(oracle, case):
         assert ok and nbad == 0, (case, vt, mad, maxref)
 
 
+TWO_BLOCKS = {(256, 32, 8, 2053, 128, 1), (192, 64, 12, 1000, 96, 1), (192, 64, 12, 1001, 97, 0),
+              (128, 2, 1, 32700, 40, 0), (64, 16, 16, 5000, 64, 1)}
+
+
 @pytest.mark.parametrize("case", [
-    # Hq, Hkv, Sq, Sk, D, causal: decode with two 16-row blocks per workgroup and its limits
+    # Hq, Hkv, Sq, Sk, D, causal: three and four 16-row blocks per kv head, one per workgroup
     (256, 32, 8, 517, 128, 1),   # four blocks, a five-key last tile
     (192, 64, 12, 400, 96, 1),   # three blocks, the last of 4 rows
     (192, 64, 12, 401, 97, 0),   # unaligned
-    (64, 1, 1, 16500, 40, 0),    # one kv head: the cap of 64 splits
+    (64, 1, 1, 16500, 40, 0),    # one kv head: 65 splits
     (64, 16, 16, 1024, 64, 1),
+    # and two per workgroup (TWO_BLOCKS)
+    (256, 32, 8, 2053, 128, 1), (192, 64, 12, 1000, 96, 1), (192, 64, 12, 1001, 97, 0),
+    (128, 2, 1, 32700, 40, 0),   # the cap of 64 splits
+    (64, 16, 16, 5000, 64, 1),
     # merges: splits of 3 to 64, column counts that end inside a 4-float piece
     (2, 2, 1, 300, 7, 0), (5, 1, 1, 1500, 101, 0), (8, 8, 1, 4100, 256, 0), (1, 1, 1, 8192, 250, 0),
     (3, 1, 4, 1030, 66, 1), (512, 128, 4, 1000, 128, 1),
 ])
 def test_decode_groups_and_merges(oracle, case):
     Hq, Hkv, Sq, Sk, D, causal = case
-    print("case", case, ts.attn_flash_plan(Hq, Hkv, Sq, Sk, D, causal), flush=True)
+    plans = [ts.attn_flash_plan(Hq, Hkv, Sq, Sk, D, causal, v_prepacked=vt) for vt in (0, 1)]
+    print("case", case, plans, flush=True)
+    if ts.device_info()["cus"] == 256:
+        for p in plans:
+            assert (", 2 blocks" in p[0][0]) == (case in TWO_BLOCKS), p
     Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, 777 + D)
     Vt = np.ascontiguousarray(V.reshape(Hkv, Sk, D).transpose(0, 2, 1)).ravel()
     rows = oracle.ref_rowset(Sq, 16)
@@ -169,7 +181,7 @@ def test_decode_groups_and_merges(oracle, case):
     (4, 2, 1, 3, 2, 0, 1, ", short", ", short"),
     (8, 2, 3, 777, 7, 1, 0, ", short", ", short"),
     (64, 64, 1, 2309, 7, 0, 3, ", short", ", short"),
-    (256, 4, 1, 8200, 5, 0, 0, ", short, 2 blocks", ", short, 2 blocks"),
+    (256, 4, 1, 16500, 5, 0, 0, ", short, 2 blocks", ", short, 2 blocks"),
     (4, 2, 1, 7, 100, 0, 0, "<128, ", ", short"),
     (4, 2, 2, 7, 200, 1, 0, "<256, ", ", short"),
     # the staged V^T kernel's limits: D > 32, more than two 128-key steps per part

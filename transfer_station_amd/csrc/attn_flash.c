@@ -42,7 +42,6 @@ int attn_hip_static_scratch(void **ptr, size_t *bytes);
  * decode path caps its split count at ATTN_SLOTS / (Hq*Sq) and runs unsplit below 2, as does
  * the key split of an under-filled prefill grid, and the causal prefill splits the key range of
  * its heavier query tiles only when their rows fit. */
-#define ATTN_SLOTS 65536
 #define ATTN_SUB_ALIGN 256
 
 static size_t align_up(size_t x, size_t a) { return (x + a - 1) & ~(a - 1); }
@@ -157,35 +156,6 @@ static int attn_use_decode(int Hkv, int group, int Sq) {
     return rows <= ATTN_DECODE_MAX_ROWS && Hkv < attn_hip_device_cus();
 }
 
-static void attn_decode_split(int Hq, int Hkv, int Sq, int Sk, int nrb, int dp, int *nsplit_o,
-                              int *kps_o) {
-    long rows = (long)Hq * Sq;
-    long cap = ATTN_SLOTS / (rows > 0 ? rows : 1);
-    /* Up to D = 128 one workgroup serves the row blocks of a key range, two of them or (at half
-     * the workgroups, one wave per SIMD) four. */
-    /* One workgroup per (kv head, split, group of row blocks). */
-    const int per = attn_decode_blocks(nrb, dp, Hkv, Sk);
-    const long wgs = (long)Hkv * ((nrb + per - 1) / per);
-    long want = (ATTN_DECODE_TARGET_WG + wgs - 1) / wgs;
-    /* Grouped blocks: no more than the 64 splits that one merge wave covers. */
-    if (per > 1 && want > 64)
-        want = 64;
-    long by_len = (Sk + ATTN_DECODE_MIN_KEYS - 1) / ATTN_DECODE_MIN_KEYS;
-    long ns = want;
-    if (ns > by_len)
-        ns = by_len;
-    if (ns > cap)
-        ns = cap;
-    if (ns < 2)
-        ns = 1;
-    /* keys per split: a multiple of 128 covering Sk in ns pieces */
-    long kps = (Sk + ns - 1) / ns;
-    kps = (kps + ATTN_DECODE_MIN_KEYS - 1) / ATTN_DECODE_MIN_KEYS * ATTN_DECODE_MIN_KEYS;
-    ns = (Sk + kps - 1) / kps;
-    *nsplit_o = (int)ns;
-    *kps_o = (int)kps;
-}
-
 static int attn_dp_for_d(int D) { return (D <= 64) ? 64 : (D <= 128 ? 128 : 256); }
 
 /* ---- timing events (only when the caller asks for tm) ------------------------------------- */
@@ -238,17 +208,17 @@ static void attn_run(const char *who, const uint16_t *Q, const uint16_t *K, cons
     }
     if (attn_use_decode(Hkv, group, Sq)) {
         const int nrb = (group * Sq + ATTN_DECODE_ROWS - 1) / ATTN_DECODE_ROWS;
-        int nsplit, kps;
-        attn_decode_split(Hq, Hkv, Sq, Sk, nrb, dp, &nsplit, &kps);
+        const struct attn_decode_cut cut = attn_decode_cut_of(Hq, Hkv, Sq, Sk, nrb, dp);
         struct attn_carve cv = {NULL, NULL, NULL};
         attn_layout(scratch, D, &cv);
         attn_hip_check(attn_hip_launch_decode(Q, K, V, O, cv.m, cv.l, cv.acc, Hq, Hkv, Sq, Sk, D,
-                                              causal ? 1 : 0, vec, vt, dp, c, nsplit, kps, nrb,
-                                              st),
+                                              causal ? 1 : 0, vec, vt, dp, c, cut.nsplit, cut.kps,
+                                              nrb, st),
                        who);
-        if (nsplit > 1)
+        if (cut.nsplit > 1)
             attn_hip_check(
-                attn_hip_launch_merge(cv.m, cv.l, cv.acc, O, Hq * Sq, D, nsplit, c, Sq, st), who);
+                attn_hip_launch_merge(cv.m, cv.l, cv.acc, O, Hq * Sq, D, cut.nsplit, c, Sq, st),
+                who);
     } else {
         struct attn_carve cv = {NULL, NULL, NULL};
         attn_layout(scratch, D, &cv);

@@ -3799,7 +3799,7 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
     if (nblk <= 0 || nblk > 0x7fffffffL)
         return hipErrorInvalidValue;
     const bool ntl = decode_nt_loads(nrb, kps);
-    const int blocks = attn_decode_blocks(nrb, DP, Hkv, Sk);
+    const int blocks = attn_decode_cut_of(Hq, Hkv, Sq, Sk, nrb, DP).blocks;
     // The staged V^T kernel, for one row block per workgroup and more than one 128-key step: its
     // pipeline fills over five barrier intervals (8 kv heads over 776 keys in one-step splits 10.3 us,
     // attn_decode_kernel straight from V^T 8.2; over 777 keys 14.2 and 10.0; two steps and up it is
