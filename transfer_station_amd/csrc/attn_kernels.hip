@@ -2569,8 +2569,7 @@ __global__ __launch_bounds__(256, DP == 256 && VT && AL == 2 ? 1 : 2) void attn_
     }
 }
 
-// Decode from V^T ([Hkv][D][Sk], D % 8 == 0, Sk % 8 == 0, 16-byte aligned tensors, DP of 64 or
-// 128): attn_decode_kernel's workgroups, rows, key order, S MFMAs and softmax, with the V^T
+// Decode from V^T ([Hkv][D][Sk], DP of 64 or 128): attn_decode_kernel's workgroups, rows, key order, S MFMAs and softmax, with the V^T
 // operand staged through LDS by LDS-DMA. HBM serves pieces of strided rows faster the longer
 // the piece: 128 rows 8 KB apart read in 256-byte pieces stream at about 4.7 TB/s, in 1 KB
 // pieces at about 5.9 TB/s (contiguous: 6.2). The kernel therefore walks the keys in groups of
@@ -2583,7 +2582,12 @@ __global__ __launch_bounds__(256, DP == 256 && VT && AL == 2 ? 1 : 2) void attn_
 // kernels' outputs are bit-identical. The 16-byte chunks of a tile row e sit at slot
 // c ^ (e % 16), so the 16 lanes of an operand read (16 d rows, one key chunk) hit 16 distinct
 // bank groups. NTL: K loads and V^T DMA are non-temporal (decode_nt_loads decides).
-template <int DP, bool CAUSAL, bool NTL, bool UA>
+// UA: 0 tensors with the 16-byte vector layout; 1 and 2 without, their V^T pieces loaded into
+// registers and put into LDS at the interval's end: 1 for D % 8 == 0, whose K and Q rows end with a
+// piece, 2 for other D, whose last pieces are shifted once they are waited for. One instance for both
+// cost D % 8 == 0 2-4%: 16 sequences of 8 kv heads over 4001 keys at D = 128 52.7 us, now 51.3; D = 100
+// 50.3 with the shift at the load, now 45.6.
+template <int DP, bool CAUSAL, bool NTL, int UA>
 __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     const uint16_t *__restrict__ V, float *__restrict__ O, float *__restrict__ pm,
@@ -2618,16 +2622,24 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
 
     bf16x8 qb[DP / 32];
     const size_t qrow = (size_t)h * Sq + qi;
+    // Columns [col, col+8) of row `row` of H, zeros if !ok or past D. UA = 2: columns that reach
+    // past D are trimmed where they are used (trim_piece).
+    auto row8 = [&](const uint16_t *H, size_t row, int col, bool ok, auto NT)
+        __attribute__((always_inline)) {
+        constexpr bool kN = decltype(NT)::value;
+        if constexpr (UA == 0)
+            return load_row8<kN>(H, row, col, D, ok);
+        if (!ok || col >= D)
+            return zero4();
+        return load16_any<kN>(H + row * D + (UA == 2 ? min(col, D - 8) : col));
+    };
     u32x4 qr[DP / 32];
 #pragma unroll
     for (int kk = 0; kk < DP / 32; ++kk)
-        qr[kk] = UA ? load_piece(Q + qrow * D, kk * 32 + grp * 8, D, kk * 32 + 32)
-                    : load_row8(Q, qrow, kk * 32 + grp * 8, D, rvalid);
+        qr[kk] = row8(Q, qrow, kk * 32 + grp * 8, rvalid, std::false_type{});
 #pragma unroll
     for (int kk = 0; kk < DP / 32; ++kk)
-        qb[kk] = as_bf16x8(!UA      ? qr[kk]
-                           : rvalid ? trim_piece(qr[kk], kk * 32 + grp * 8, D, kk * 32 + 32)
-                                    : zero4());
+        qb[kk] = as_bf16x8(UA == 2 ? trim_piece(qr[kk], kk * 32 + grp * 8, D, kk * 32 + 32) : qr[kk]);
     const int lim = CAUSAL ? min(Sk - 1, Sk - Sq + qi) : Sk - 1;
 
     float m_run = kNegInf, l_run = 0.f;
@@ -2700,20 +2712,18 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
             const int key = tb + 8 * (r16 >> 2) + 4 * t + (r16 & 3);
 #pragma unroll
             for (int kk = 0; kk < DP / 32; ++kk)
-                dst[t][kk] =
-                    UA ? load_piece<NTL>(Kh + (size_t)min(key, k1 - 1) * D, kk * 32 + grp * 8, D,
-                                         kk * 32 + 32)
-                       : load_row8<NTL>(Kh, (size_t)key, kk * 32 + grp * 8, D, key < k1);
+                dst[t][kk] = row8(Kh, (size_t)key, kk * 32 + grp * 8, key < k1,
+                                  std::integral_constant<bool, NTL>{});
         }
     };
-    // src, as load_k put it there, into ka.
-    auto take_k = [&](const u32x4 (&src)[2][DP / 32]) {
+    // kn, once it is waited for, into ka.
+    auto take_k = [&]() {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int kk = 0; kk < DP / 32; ++kk)
-                ka[t][kk] = UA ? trim_piece(src[t][kk], kk * 32 + grp * 8, D, kk * 32 + 32)
-                               : src[t][kk];
+                ka[t][kk] = UA == 2 ? trim_piece(kn[t][kk], kk * 32 + grp * 8, D, kk * 32 + 32)
+                                    : kn[t][kk];
     };
 
     bf16x8 pkp[4], pkc[4]; // softmax weights of the previous / current group's steps
@@ -2721,8 +2731,13 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
     int livep = 0, livec = 0; // bit st: step st of the previous / current group was scored
     int buf = 0;
     if (ngr > 0) {
-        load_k(k0 + step_of(0) * 128 + w * 32, kn);
-        take_k(kn);
+        const int tb = k0 + step_of(0) * 128 + w * 32;
+        if constexpr (UA == 2) {
+            load_k(tb, kn);
+            take_k();
+        } else {
+            load_k(tb, ka);
+        }
     }
     for (int j = 0; j <= ngr; ++j) {
         const bool cur = j < ngr;
@@ -2806,7 +2821,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_vt_kernel(
             // The next step's K fragments (waiting for them here leaves the loads in flight
             // under both halves of the interval).
             if (tbn >= 0)
-                take_k(kn);
+                take_k();
             if (UA && (i < 3 ? j > 0 : cur))
                 put_tile(i < 3 ? j - 1 : j, buf ^ 1);
             buf ^= 1;
@@ -3814,9 +3829,9 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
             (vec ? (long)D * Sk * 2 < 0x7fffffffL : D > 32 && kps > 2 * ATTN_DECODE_MIN_KEYS))
             return with_flag(causal != 0, [&](auto CA) {
                 return with_flag(ntl, [&](auto NT) {
-                    return with_flag(vec == 0, [&](auto UAF) {
-                        constexpr bool kC = decltype(CA)::value, kN = decltype(NT)::value,
-                                       kU = decltype(UAF)::value;
+                    auto launch = [&](auto UAF) {
+                        constexpr bool kC = decltype(CA)::value, kN = decltype(NT)::value;
+                        constexpr int kU = decltype(UAF)::value;
                         if (t_plan)
                             plan_note(dim3((unsigned)nblk), dim3(256),
                                       "attn_decode_vt_kernel<%d, %s, %s%s> nsplit=%d nrb=%d", DP,
@@ -3827,7 +3842,10 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
                                                pm, pl, pacc, Hq, Hkv, Sq, Sk, D, c, nsplit, kps,
                                                nrb);
                         return hipGetLastError();
-                    });
+                    };
+                    return vec          ? launch(std::integral_constant<int, 0>{})
+                           : D % 8 == 0 ? launch(std::integral_constant<int, 1>{})
+                                        : launch(std::integral_constant<int, 2>{});
                 });
             });
     auto go = [&](auto NB) {
