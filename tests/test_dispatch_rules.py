@@ -93,3 +93,20 @@ def test_decode_row_blocks_per_workgroup(case):
 def test_kernels_by_shape(case):
     Hq, Hkv, Sq, Sk, D, causal, vt, want = case
     assert plan(Hq, Hkv, Sq, Sk, D, causal, vt)[0][0].startswith(want), case
+
+
+@pytest.mark.parametrize("case", [
+    # Hq, Hkv, Sq, Sk, D, two workgroups per CU instead of three
+    (1600, 400, 1, 3560, 96, 1),    # 800 workgroups: 3 per CU would leave a round of 32
+    (1600, 400, 1, 2047, 96, 1),    # 1024 keys each
+    (1600, 400, 1, 1792, 96, 0),    # 896 keys each
+    (1536, 384, 1, 3560, 128, 0),   # 768: three full per CU
+    (2048, 512, 1, 4096, 128, 0),
+    (3200, 800, 1, 3560, 128, 1),   # unsplit
+    (6400, 1600, 1, 3560, 128, 0),  # 1600: no better filled by twos
+    (1600, 400, 1, 3560, 64, 0),    # other instances
+    (1600, 400, 1, 3560, 160, 0),
+])
+def test_decode_rounds_of_two_per_cu(case):
+    Hq, Hkv, Sq, Sk, D, two = case
+    assert ("two-per-cu=1" in plan(Hq, Hkv, Sq, Sk, D, 0)[0][1].split()) == bool(two), case

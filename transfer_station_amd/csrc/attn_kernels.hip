@@ -3848,6 +3848,17 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
                                         : launch(std::integral_constant<int, 2>{});
                 });
             });
+    // The aligned row-major instance at DP = 128 keeps three workgroups on a CU. A grid a little past
+    // three per CU then ends in a round of few workgroups, which long key ranges feel; where rounds of
+    // two per CU are a fifth better filled, LDS that nobody uses holds the third one back. 400 heads x
+    // 3560 keys at D = 96 (800 workgroups) two per CU 101.3, three 109.5, this 100.7 us; 420 x 6000
+    // 173, 180, 174; at under 1024 keys per workgroup three stay ahead (400 x 1000 35.9, 35.3).
+    auto hold_third = [&](long n) -> unsigned {
+        const long c2 = 2L * device_cus(), c3 = 3L * device_cus();
+        const bool two = n > c3 && kps >= 1024 &&
+                         6 * ((n + c2 - 1) / c2 * c2) < 5 * ((n + c3 - 1) / c3 * c3);
+        return two ? 17408 : 0; // with the kernel's 37376 bytes, three do not fit 160 KB
+    };
     auto go = [&](auto NB) {
         constexpr int NRB = decltype(NB)::value;
         const int ng = (nrb + NRB - 1) / NRB; // row block groups
@@ -3856,14 +3867,16 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
             constexpr bool kC = decltype(CA)::value, kT = decltype(VTF)::value,
                            kN = decltype(NT)::value;
             constexpr int kA = decltype(ALF)::value;
+            constexpr bool kThree = DP == 128 && kA == 1 && !kT && NRB == 1;
             if (t_plan)
                 plan_note(dim3((unsigned)n), dim3(256),
-                          "attn_decode_kernel<%d, %s, %s, %s, %s%s%s> nsplit=%d nrb=%d", DP,
+                          "attn_decode_kernel<%d, %s, %s, %s, %s%s%s> nsplit=%d nrb=%d%s", DP,
                           tf(kC), tf(kA == 1), tf(kT), tf(kN), kA == 2 ? ", short" : "",
-                          NRB == 2 ? ", 2 blocks" : "", nsplit, nrb);
+                          NRB == 2 ? ", 2 blocks" : "", nsplit, nrb,
+                          kThree && hold_third(n) ? " two-per-cu=1" : "");
             else
                 hipLaunchKernelGGL((attn_decode_kernel<DP, kC, kA, kT, kN, NRB>),
-                                   dim3((unsigned)n), dim3(256), 0, st, Q, K, V, O, pm, pl, pacc,
+                                   dim3((unsigned)n), dim3(256), kThree ? hold_third(n) : 0, st, Q, K, V, O, pm, pl, pacc,
                                    Hq, Hkv, Sq, Sk, D, c, nsplit, kps, ng);
             return hipGetLastError();
         };
