@@ -98,6 +98,7 @@ def test_kernels_by_shape(case):
 @pytest.mark.parametrize("case", [
     # Hq, Hkv, Sq, Sk, D, two workgroups per CU instead of three
     (1600, 400, 1, 3560, 96, 1),    # 800 workgroups: 3 per CU would leave a round of 32
+    (1600, 400, 1, 3560, 99, 1),    # without the vector layout
     (1600, 400, 1, 2047, 96, 1),    # 1024 keys each
     (1600, 400, 1, 1792, 96, 0),    # 896 keys each
     (1536, 384, 1, 3560, 128, 0),   # 768: three full per CU

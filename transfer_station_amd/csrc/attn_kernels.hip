@@ -3848,8 +3848,8 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
                                         : launch(std::integral_constant<int, 2>{});
                 });
             });
-    // The aligned row-major instance at DP = 128 keeps three workgroups on a CU. A grid a little past
-    // three per CU then ends in a round of few workgroups, which long key ranges feel; where rounds of
+    // The row-major instances at DP = 128 keep three workgroups on a CU. A grid a little past three
+    // per CU then ends in a round of few workgroups, which long key ranges feel; where rounds of
     // two per CU are a fifth better filled, LDS that nobody uses holds the third one back. 400 heads x
     // 3560 keys at D = 96 (800 workgroups) two per CU 101.3, three 109.5, this 100.7 us; 420 x 6000
     // 173, 180, 174; at under 1024 keys per workgroup three stay ahead (400 x 1000 35.9, 35.3).
@@ -3867,7 +3867,7 @@ hipError_t launch_decode_d(const uint16_t *Q, const uint16_t *K, const uint16_t 
             constexpr bool kC = decltype(CA)::value, kT = decltype(VTF)::value,
                            kN = decltype(NT)::value;
             constexpr int kA = decltype(ALF)::value;
-            constexpr bool kThree = DP == 128 && kA == 1 && !kT && NRB == 1;
+            constexpr bool kThree = DP == 128 && kA != 2 && !kT && NRB == 1;
             if (t_plan)
                 plan_note(dim3((unsigned)n), dim3(256),
                           "attn_decode_kernel<%d, %s, %s, %s, %s%s%s> nsplit=%d nrb=%d%s", DP,
