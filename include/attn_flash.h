@@ -17,7 +17,7 @@
  *     path and for prefills too small to fill the GPU, whose key ranges are split (34 MB at
  *     D = 128).
  *   - bk is validated and sizes the scratch but does not pick the key tile: the GPU's
- *     tile is fixed by D (128 keys up to D = 128, 64 beyond), so O is bit-identical at
+ *     tile (32, 64 or 128 keys) follows from the other arguments, so O is bit-identical at
  *     every bk. The reference's result is bk-invariant within its tolerance.
  *
  * Layouts (row-major, bf16 stored as uint16_t bits, O fp32):

@@ -227,7 +227,7 @@ def test_head_dim_sweep(oracle, D):
         check(oracle, "D sweep", Q, K, V, Hq, Hkv, Sq, 150, D, 1, 64)
 
 
-# ---- head dims past 128 (up to ATTN_D_MAX = 256): the general prefill kernel on 32-key tiles
+# ---- head dims past 128 (up to ATTN_D_MAX = 256): prefill on 192- and 256-wide tiles
 # and the 256-wide decode kernel ----------------------------------------------------------------
 @pytest.mark.parametrize("shape", [
     (8, 2, 300, 700, 256, 1, 64, 0),     # GQA prefill, causal, bk 64
@@ -237,9 +237,9 @@ def test_head_dim_sweep(oracle, D):
     (8, 2, 300, 640, 256, 1, 128, 1),    # prefill from V^T
     (8, 2, 1, 2048, 256, 0, 128, 1),     # decode from V^T
     (8, 2, 200, 500, 224, 1, 16, 0),     # causal key split, D = 224, bk 16
-    (6, 3, 130, 70, 200, 1, 128, 0),     # general kernel (D % 8 != 0)
+    (6, 3, 130, 70, 200, 1, 128, 0),     # Sq > Sk: the first rows see no key
 ], ids=["prefill-causal", "prefill-ragged", "decode", "decode-d192", "prefill-vt", "decode-vt",
-        "bk16-split-d224", "general-d200"])
+        "bk16-split-d224", "sq>sk-d200"])
 def test_head_dim_256(oracle, shape):
     Hq, Hkv, Sq, Sk, D, causal, bk, vt = shape
     Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, SEED0 + 256 + Sk)
@@ -333,7 +333,7 @@ def test_batch_fold_bitwise_and_determinism():
     (8, 1, 1024, 8192, 128, 0, 8),   # MQA
     (16, 4, 256, 4096, 64, 0, 0),    # D = 64 (software-pipelined tiles inside each part)
     (8, 2, 512, 1024, 128, 1, 0),    # causal, Sk - Sq == Sq: the shortest tiles get empty parts
-    (6, 3, 200, 777, 36, 0, 0),      # general kernel (D % 8 != 0): no split, the same answer
+    (6, 3, 200, 777, 36, 0, 0),      # unaligned tiles (D % 8 != 0)
 ])
 def test_prefill_key_split(oracle, Hq, Hkv, Sq, Sk, D, causal, ref_cap):
     """Grids that fill at most half of one round of resident workgroups split each query tile's
@@ -501,7 +501,7 @@ def test_key_permutation_invariance(oracle):
 def test_bk_invariance(oracle, D, Sk):
     """The reference's result is bk-invariant within the tolerance (README:354-357). Here bk is
     validated and sizes the scratch but never picks the key tile, so O is bit-identical at
-    every bk, on the fast, the D > 128 and the general (D % 8 != 0) kernels alike."""
+    every bk, at D <= 128 and past it, with and without ragged key counts alike."""
     Hq, Hkv, Sq = 8, 2, 300
     Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, 14)
     base = ts.run_attention(Q, K, V, Hq, Hkv, Sq, Sk, D, 1, 128)
@@ -513,15 +513,15 @@ def test_bk_invariance(oracle, D, Sk):
 
 # ---- the other entry points ------------------------------------------------------------------------
 @pytest.mark.parametrize("Hkv,Sk,D,offset", [
-    (3, 77, 40, 0),     # element-wise path (Sk % 8 != 0)
+    (3, 77, 40, 0),     # pieces at element alignment (Sk % 8 != 0)
     (3, 80, 40, 0),     # 16-byte path, partial 64-column tile
     (1, 200, 64, 0),    # 16-byte path, partial key tile (72 of 128 keys)
     (2, 136, 96, 0),    # 16-byte path, one 8-key chunk in the last key tile, 32 of 64 columns
     (2, 4096, 128, 0),  # 16-byte path, full tiles
     (2, 8, 8, 0),       # 16-byte path, one chunk per row
-    (2, 64, 64, 2),     # misaligned by one element: element-wise path
+    (2, 64, 64, 2),     # misaligned by one element
     (65535 + 7, 8, 8, 0),  # more kv heads than one launch's z range: two launches
-    (65535 + 2, 9, 7, 0),  # the same on the element-wise path
+    (65535 + 2, 9, 7, 0),  # the same with rows shorter than a piece
 ])
 def test_pack_v_full_transposes_exactly(Hkv, Sk, D, offset):
     rng = np.random.default_rng(Sk * 1000 + D)
@@ -542,8 +542,8 @@ def test_pack_v_full_transposes_exactly(Hkv, Sk, D, offset):
 # The reference changes only V's stride when V is pre-packed, so the math is identical. Here the
 # V^T operand of the P.V MFMA holds the same values in the same positions either way, so O is
 # bit-identical whenever both layouts run the same kernel. They do not when D % 8 == 0 and
-# Sk % 8 != 0 (a V^T row is then not 16-byte aligned and the prefill takes the general kernel
-# while row-major V takes the fast one): those cases are held to the oracle tolerance only.
+# Sk % 8 != 0 (a V^T row is then not 16-byte aligned and the prefill takes the unaligned instances
+# while row-major V takes the aligned ones): those cases are held to the oracle tolerance only.
 VT_CASES = [
     # name, Hq, Hkv, Sq, Sk, D, causal, bk
     ("fast D128 partial tile", 8, 2, 300, 1000, 128, 0, 128),
@@ -555,9 +555,9 @@ VT_CASES = [
     ("fast D96 causal", 8, 2, 300, 640, 96, 1, 128),
     ("fast D80 bk64", 8, 4, 200, 512, 80, 0, 64),
     ("fast D40 bk32", 6, 3, 130, 72, 40, 1, 32),
-    ("general D128 Sk%8!=0", 8, 2, 200, 333, 128, 0, 128),
-    ("general D64 Sk%8!=0 causal", 4, 1, 64, 77, 64, 1, 32),
-    ("general D7", 4, 2, 40, 50, 7, 0, 64),
+    ("unaligned D128 Sk%8!=0", 8, 2, 200, 333, 128, 0, 128),
+    ("unaligned D64 Sk%8!=0 causal", 4, 1, 64, 77, 64, 1, 32),
+    ("short rows D7", 4, 2, 40, 50, 7, 0, 64),
     ("decode Sq=1 split", 8, 2, 1, 2048, 128, 0, 128),
     ("decode Sq=2 causal", 4, 1, 2, 1000, 64, 1, 128),
     ("decode Sk%8!=0", 8, 1, 2, 4099, 128, 1, 128),
@@ -877,7 +877,7 @@ RANDOM_CASES = _random_cases(40, 0x5EED)
 def test_random_shapes(oracle, case):
     """Seeded random shapes (GQA group 1-16, Sq 1-700, Sk 1-1500 with and without Sk % 8,
     D in {32, 64, 80, 96, 128}, causal or not, bk 16-512, row-major V or V^T) against the
-    oracle: decode, prefill fast and general kernels, tails and the causal key split."""
+    oracle: decode, aligned and unaligned prefill, tails and the causal key split."""
     i, Hq, Hkv, Sq, Sk, D, causal, bk, vt = case
     Q, K, V = ts.synth_normal_qkv(Hq, Hkv, Sq, Sk, D, SEED0 + 1000 + i)
     if vt:
@@ -890,7 +890,7 @@ def test_random_shapes(oracle, case):
 
 
 # ---- a kv head past 2 GiB: K and V exceed a buffer's 31-bit range, so the prefill takes the
-# general kernel (64-bit element offsets), and decode and the V^T path read past 2 GiB as well --
+# unaligned instances (64-bit tile bases), and decode and the V^T path read past 2 GiB as well --
 def _spread_bf16(n, seed):
     """n finite bf16 values: random sign and mantissa, magnitude in [2^-7, 2), so that an offset
     that wrapped at 2^31 bytes would read different values."""
@@ -909,7 +909,7 @@ def kv_over_2gib():
 
 
 @pytest.mark.parametrize("Hq,Sq,causal,prepack", [
-    (2, 40, 1, False),   # prefill, general kernel, causal
+    (2, 40, 1, False),   # prefill, unaligned instance, causal
     (2, 1, 0, False),    # split-K decode
     (2, 40, 0, True),    # prefill from V^T packed on the device
 ], ids=["prefill-causal", "decode", "prefill-vt"])
@@ -922,7 +922,7 @@ def test_kv_head_over_2gib(oracle, kv_over_2gib, Hq, Sq, causal, prepack):
 
 
 def _random_cases_wide(n, seed):
-    """Head dims past 128 (odd ones on the general kernel), short query blocks that pack the
+    """Head dims past 128 (odd ones on the unaligned tiles), short query blocks that pack the
     GQA heads' rows, and many kv heads (the decode / packed-prefill choice)."""
     rng = np.random.default_rng(seed)
     cases = []

@@ -169,8 +169,8 @@ static void attn_events(void) {
 }
 
 /* Argument checks shared by both attention entry points. bk keeps the reference's contract
- * (validated here, scratch sized with it), but the key tile is the hardware's: 128 keys up to
- * D = 128, 64 beyond, whatever bk says. In the reference bk is a cache-blocking knob whose
+ * (validated here, scratch sized with it), but the key tile is the kernel's: 32, 64 or 128
+ * keys by head dim, alignment and workgroup, whatever bk says. In the reference bk is a cache-blocking knob whose
  * result is bk-invariant within the tolerance (README.md:354-357); on the GPU a smaller tile is
  * only slower. */
 static void attn_check_args(const char *who, const uint16_t *Q, const uint16_t *K,

@@ -272,7 +272,7 @@ __device__ __forceinline__ void lds_wave_fence() {
 // ------------------------------------------------------------------------------------------
 // Prefill, D <= DP (64, 96, 128, 192 or 256); the head-dim columns D .. DP-1 are zero in the tiles and
 // in Q, and are never stored. NW waves per workgroup (8: 256 query rows, two waves per SIMD; 4 on
-// grids too small to fill the GPU, and always past DP = 128, where one wave per SIMD holds O and Q);
+// grids too small to fill the GPU; past DP = 128 4 waves are one per SIMD, which holds O and Q);
 // wave w owns 32 query rows. Per key tile of KT keys (one online-softmax update per tile):
 //   S^T[key][q] = K_tile . Q^T     (v_mfma_f32_32x32x16_bf16, A = K rows from LDS, B = Q regs)
 //   each lane holds one query (q = lane%32) and 16 keys per 32-key sub-tile, so the row max is
@@ -406,7 +406,9 @@ constexpr int prefill_wg_per_cu(int DP, int KT, int NW) {
 // with the sum test, which was 8% faster). Same box, element-wise loads before -> now: 24 heads of
 // 1000 rows over 2003 keys, D = 100, V^T with its pack 249 -> 57 us; 64 heads at 2k, D = 128, V^T
 // of 2003 keys 950 -> 172 us; D = 100 causal 524 -> 118 us (aligned, D = 128: 126 us non-causal).
-// UA = 2: rows shorter than a piece (D < 8), read element by element.
+// UA = 2: rows shorter than a piece (D < 8), a row per 16-byte load with the rows behind it masked off.
+// Against element-wise loads: 128 heads x 20 rows over 1720 keys at D = 7 66 -> 46 us, 8 heads x 317 rows
+// over 817 keys 35 -> 26; calls of one tile from V^T stay 0.3-0.8 us above (4.5-7 us).
 template <int DP, int KT, int NW, bool CAUSAL, bool VT, bool KH, int UA>
 __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_prefill_fast_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
@@ -414,7 +416,7 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     float c, int nqt, int split_first, float *__restrict__ pm, float *__restrict__ pl,
     float *__restrict__ pacc, int prows, int pack, int pair_r, int pipe, int nsplit, int nwg,
     int hsplit) {
-    // D <= DP, D % 8 == 0: head-dim columns D .. DP-1 of the tiles and of Q are zero.
+    // D <= DP: head-dim columns D .. DP-1 of the tiles and of Q are zero.
     static_assert(DP % 32 == 0 && KT % 32 == 0, "tile shape");
     static_assert(!KH || (KT == 128 && ((NW == 8 && DP >= 64) || (NW == 12 && DP == 64 && !CAUSAL))),
                   "key halves: 8 waves (or 12 at DP = 64), 128-key tiles");
@@ -427,7 +429,9 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
     // latency then runs under the other's MFMAs, and a tile is read from L2 for 256 rows. Same
     // box, 4 -> 8 waves, 64 heads at 2k: D = 256 282 -> 232 us (1185 TFLOP/s), causal 160 -> 136, V^T
     // 322 -> 238, D = 192 220 -> 184; unaligned, D = 189 over 2003 keys 530 -> 253, D = 250 at 1000
-    // rows 307 -> 154. Bound as the 8-wave kernels at DP = 128 are: LDS reads beside the MFMAs.
+    // rows 307 -> 154. Neither unit is full (counters at D = 256: MFMA busy 50% of the clocks, no LDS
+    // conflicts): a tile's LDS reads take about as long as its MFMAs, and two waves per SIMD, in step
+    // through a barrier per tile, overlap them in part.
     constexpr bool kRing = DP > 128 && NW == 8;
     constexpr int RD = !kRing ? 1 : DP < 256 ? 4 : UA ? 2 : VT ? 3 : 4;
     constexpr bool kPipe = DP <= 64 && (!KH || NW == 12) && !UA;
@@ -2289,8 +2293,10 @@ __device__ __forceinline__ void decode_merge(const float *om, const float (*red_
 // the load and MFMA latencies: 36.9 us), two blocks where there are two (24-32 heads' rows over 2000
 // keys at D = 64 8.1 -> 9.0 us: half the workgroups), the next step's loads issued a step ahead
 // (+5 to +12%, the registers take a wave per SIMD).
-// Two waves per SIMD are asked for; the 138 registers at D = 128 allow three (172 with no bound:
-// c2 162.4 -> 160 us, D = 256 with 8 kv heads 18.7 -> 14.9).
+// Two waves per SIMD are asked for (one for AL = 2 from V^T at DP = 256, which hardly any call reaches):
+// the 137-165 registers at DP = 128 then allow three, where no bound took 172-185 (512 kv heads x 4096
+// keys 162.6 -> 159.6 us, 200 x 300 14.9 -> 12.3; 8 kv heads at D = 256 17.9 -> 13.1). No instance
+// spills; at DP = 256 that takes kLate.
 template <int DP, bool CAUSAL, int AL, bool VT, bool NTL, int NRB>
 __global__ __launch_bounds__(256, DP == 256 && VT && AL == 2 ? 1 : 2) void attn_decode_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
@@ -2937,7 +2943,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
 // splits (a row per 16 lanes, or per wave past 16 splits), then NL splits' columns per thread
 // without a branch, and only then the weights, which go through LDS, as the groups' sums do. One
 // wave per row reading its splits one by one took 7.2 us for 32 rows x 64 splits at D = 128 (8
-// workgroups); decode over 32768 keys 34.6 -> 30.3 us with this layout. A wave per row for the
+// workgroups); decode over 32768 keys 34.5 -> 29.9 us with this layout. A wave per row for the
 // weights, and branches around the loads, cost short merges 1 to 2 us: 202 rows x 3 splits at
 // D = 32 5.3 us, 10144 rows x 3 at D = 128 8.8.
 constexpr int kMergeWaveMaxSplit = 64;
@@ -3706,8 +3712,9 @@ hipError_t launch_prefill_fast_t(const uint16_t *Q, const uint16_t *K, const uin
                                                           pl, pacc, slots, st);
 }
 
-// Unaligned tensors (UA): the aligned kernels' choice of workgroup, without the persistent, head
-// split and 12-wave variants, on 64-key tiles (two staged pieces per thread and tensor at 8 waves).
+// Unaligned tensors (UA): the aligned kernels' choice of workgroup, without the persistent and 12-wave
+// variants. Key tiles: 64 keys on 4 and 8 waves at D in (64, 128] (two staged pieces per thread and
+// tensor at 8 waves), 128 at D <= 64 and for key halves, 32 past D = 128.
 template <int DP, int KT, bool CAUSAL, bool VT>
 hipError_t launch_prefill_ua(const uint16_t *Q, const uint16_t *K, const uint16_t *V, float *O,
                              int Hq, int Hkv, int Sq, int Sk, int D, float c, float *pm, float *pl,
@@ -3926,7 +3933,7 @@ extern "C" int attn_hip_launch_prefill(const uint16_t *Q, const uint16_t *K, con
     }
 }
 
-// nrb: 16-row blocks per kv head (g*Sq rows), one workgroup each.
+// nrb: 16-row blocks per kv head (g*Sq rows); attn_decode_cut_of has how many a workgroup serves.
 extern "C" int attn_hip_launch_decode(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                       float *O, float *pm, float *pl, float *pacc, int Hq,
                                       int Hkv, int Sq, int Sk, int D, int causal, int vec, int vt,
