@@ -593,10 +593,15 @@ __global__ __launch_bounds__(NW * 64, prefill_wg_per_cu(DP, KT, NW)) void attn_p
             u32x4 v = zero4();
             if constexpr (UA == 0)
                 v = load_row8(Q, qrow, col, D, rvalid);
-            else if (rvalid)
-                v = UA == 2 ? load_short(Q + qrow * D, col, D)
-                            : trim_piece(load_piece(Q + qrow * D, col, D, kk * 16 + 16), col, D,
-                                         kk * 16 + 16);
+            else if (rvalid && col < D) {
+                const uint16_t *q = Q + qrow * D;
+                if constexpr (UA == 2)
+                    v = load_short(q, col, D);
+                else if ((D & 7) != 0 && kk * 16 + 16 > D) // shifted here: once per workgroup
+                    v = drop_elems(load16_any<false>(q + min(col, D - 8)), max(col + 8 - D, 0));
+                else
+                    v = load16_any<false>(q + col);
+            }
             qb[kk] = as_bf16x8(v);
         }
     }
